@@ -478,8 +478,32 @@ int ensure_masks(sph_system* s)
     return 0;
 }
 
+// The pair counters (CNT_COPIES copies on the device): cleared before the
+// passes of a call, fetched into the pinned mirror and summed after them.
+int clear_counters(sph_system* s)
+{
+    HIPC(hipMemsetAsync(s->pair_counter, 0, sizeof(unsigned long long) * CNT_SLOTS, s->stream));
+    return 0;
+}
+
+int fetch_counters(sph_system* s)
+{
+    HIPC(hipMemcpyAsync(s->pair_counter_host, s->pair_counter,
+                        sizeof(unsigned long long) * CNT_SLOTS, hipMemcpyDeviceToHost, s->stream));
+    return 0;
+}
+
+// Counter i of the last fetch (after a stream synchronisation).
+unsigned long long counter_total(const sph_system* s, int i)
+{
+    unsigned long long t = 0;
+    for (int k = 0; k < CNT_COPIES; ++k) t += s->pair_counter_host[k * CNT_STRIDE + i];
+    return t;
+}
+
 // Grid of the pair kernels: the tiles are taken from a work queue, so a
-// grid that fills the chip is enough.
+// grid that fills the chip is enough (the launch cuts it to what the chip
+// holds of the kernel).
 int pair_grid(long long ntiles)
 {
     const long long g = std::min<long long>(ntiles, 256 * 32);
@@ -549,14 +573,18 @@ int new_handle(int precision, sph_system** out)
         s->stream = nullptr;
         rc = fail(SPH_EHIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
     }
-    if (!rc && !(rc = dalloc(s, &s->meta, META_SLOTS)) && !(rc = dalloc(s, &s->pair_counter, 4)) &&
+    if (!rc && !(rc = dalloc(s, &s->meta, META_SLOTS)) && !(rc = dalloc(s, &s->pair_counter, CNT_SLOTS)) &&
         !(rc = dalloc(s, &s->queue, NQUEUE * QSTRIDE)) &&
         !(rc = dalloc(s, &s->red_out, 4)) && !(rc = dalloc(s, &s->mask_total, 1))) {
         e = hipHostMalloc((void**)&s->meta_host, sizeof(int) * META_SLOTS, hipHostMallocDefault);
-        if (e != hipSuccess) {
-            s->meta_host = nullptr;
-            rc = fail(SPH_EHIP, std::string("hipHostMalloc: ") + hipGetErrorString(e));
+        if (e != hipSuccess) s->meta_host = nullptr;
+        if (e == hipSuccess) {
+            e = hipHostMalloc((void**)&s->pair_counter_host, sizeof(unsigned long long) * CNT_SLOTS,
+                              hipHostMallocDefault);
+            if (e != hipSuccess) s->pair_counter_host = nullptr;
         }
+        if (e != hipSuccess)
+            rc = fail(SPH_EHIP, std::string("hipHostMalloc: ") + hipGetErrorString(e));
     }
     if (!rc) {
         std::memset(s->meta_host, 0, sizeof(int) * META_SLOTS);
@@ -583,12 +611,13 @@ int destroy(sph_system* s)
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     free_particle_arrays(s);
     free_cell_arrays(s);
-    dfree(s, s->meta, META_SLOTS); dfree(s, s->pair_counter, 4); dfree(s, s->red_out, 4);
+    dfree(s, s->meta, META_SLOTS); dfree(s, s->pair_counter, CNT_SLOTS); dfree(s, s->red_out, 4);
     dfree(s, s->queue, NQUEUE * QSTRIDE);
     dfree(s, s->masks, s->mask_cap); dfree(s, s->mask_total, 1);
     dfree(s, s->kept, s->kept_cap); dfree(s, s->kept_rg, s->kept_cap);
     dfree(s, s->sysd, s->sysd_cap); dfree(s, s->sys_cnt, SYSCNT * s->sys_cnt_cap);
     if (s->meta_host) (void)hipHostFree(s->meta_host);
+    if (s->pair_counter_host) (void)hipHostFree(s->pair_counter_host);
     if (s->sys_cnt_host) (void)hipHostFree(s->sys_cnt_host);
     for (auto e : s->ev_pool) (void)hipEventDestroy(e);
     for (auto& e : s->ev_open) {
@@ -900,7 +929,7 @@ int run_steps(sph_system* s, int scheme, int nsteps)
     }
     // Tiles are taken from a work queue: the grid needs no tile count.
     const long long tiles_bound = s->tile_cap;
-    HIPC(hipMemsetAsync(s->pair_counter, 0, 3 * sizeof(unsigned long long), s->stream));
+    if ((rc = clear_counters(s))) return rc;
     int k = 0;
     const int per = scheme == SPH_SCHEME_COLLAPSE_DRY ? 1 : 2;
     if (s->use_graph && nsteps / per >= 2) {
@@ -909,9 +938,9 @@ int run_steps(sph_system* s, int scheme, int nsteps)
     }
     for (; k < nsteps; ++k)
         if ((rc = one_step(s, scheme, eos, tiles_bound))) return rc;
-    HIPC(hipMemcpyAsync(s->step_pairs, s->pair_counter, 3 * sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, s->stream));
+    if ((rc = fetch_counters(s))) return rc;
     if ((rc = sync_meta(s))) return rc;
+    for (int i = 0; i < 3; ++i) s->step_pairs[i] = counter_total(s, i);
     if (nsteps > 0) {
         s->retired_since_build = false;
         s->cells_valid = s->masks_valid = false;  // positions moved after the last build
@@ -1249,14 +1278,15 @@ int neighbour_pairs(sph_system* s, int only_slot, int64_t* pairs, int64_t cap, i
     }
     unsigned long long total = 0;
     long long* dpairs = nullptr;
-    hipError_t e = hipMemsetAsync(s->pair_counter, 0, sizeof(unsigned long long), s->stream);
-    rc = e == hipSuccess ? 0 : fail(SPH_EHIP, std::string("hipMemsetAsync: ") + hipGetErrorString(e));
+    hipError_t e = hipSuccess;
+    rc = clear_counters(s);
     if (!rc)
         rc = run_pair(s, P_COUNT, 0, 0, s->pair_counter, s->meta_host[META_NTILES],
                       SPH_KERNEL_DENSITY, MASK_TEST, flagged);
+    if (!rc) rc = fetch_counters(s);
     if (!rc) {
-        e = hipMemcpyAsync(&total, s->pair_counter, sizeof(total), hipMemcpyDeviceToHost, s->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+        e = hipStreamSynchronize(s->stream);
+        if (e == hipSuccess) total = counter_total(s, 0);
         if (e != hipSuccess) rc = fail(SPH_EHIP, std::string("pair count: ") + hipGetErrorString(e));
     }
     *n = (int64_t)total;

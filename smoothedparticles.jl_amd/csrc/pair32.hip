@@ -756,7 +756,7 @@ __global__ __launch_bounds__(64, KEPT ? Op::WAVES_KEPT : Op::WAVES) void k_pair3
     const bool kept_ok = ok && c.kept != nullptr && ld_const(c.meta + META_KEPT_OK) != 0;
     if ((load_masks && kept_ok) != KEPT) return;
     TileCursor tc;
-    tile_cursor_init(tc);
+    tile_cursor_init(c, ntiles, tc);
     // accepted pairs of all the wave's tiles, one atomic per wave
     unsigned npairs = 0;
     unsigned long long ntests = 0;
@@ -774,14 +774,14 @@ template <int ROWS, bool FLAT, bool PER, int T, bool KEPT>
 static void launch_tile_k(int op, const PairCtx& c, int grid, hipStream_t st)
 {
     switch (op) {
-    case P_DENSITY: k_pair32<ROWS, FLAT, PER, T, Density32, KEPT><<<grid, 64, 0, st>>>(c, C_RHO); break;
-    case P_DENSITY_RHO0: k_pair32<ROWS, FLAT, PER, T, Density32, KEPT><<<grid, 64, 0, st>>>(c, C_RHO0); break;
-    case P_FORCE: k_pair32<ROWS, FLAT, PER, T, Force32, KEPT><<<grid, 64, 0, st>>>(c, 0); break;
-    case P_COUNT: k_pair32<ROWS, FLAT, PER, T, Pairs32<false>, KEPT><<<grid, 64, 0, st>>>(c, 0); break;
-    case P_EMIT: k_pair32<ROWS, FLAT, PER, T, Pairs32<true>, KEPT><<<grid, 64, 0, st>>>(c, 0); break;
-    case P_DIGEST: k_pair32<ROWS, FLAT, PER, T, Digest32, KEPT><<<grid, 64, 0, st>>>(c, 0); break;
-    case P_FORCE_RHO0: k_pair32<ROWS, FLAT, PER, T, ForceRho032, KEPT><<<grid, 64, 0, st>>>(c, 0); break;
-    case P_CONTINUITY: k_pair32<ROWS, FLAT, PER, T, Continuity32, KEPT><<<grid, 64, 0, st>>>(c, 0); break;
+    case P_DENSITY: launch_resident<k_pair32<ROWS, FLAT, PER, T, Density32, KEPT>>(grid, st, c, C_RHO); break;
+    case P_DENSITY_RHO0: launch_resident<k_pair32<ROWS, FLAT, PER, T, Density32, KEPT>>(grid, st, c, C_RHO0); break;
+    case P_FORCE: launch_resident<k_pair32<ROWS, FLAT, PER, T, Force32, KEPT>>(grid, st, c, 0); break;
+    case P_COUNT: launch_resident<k_pair32<ROWS, FLAT, PER, T, Pairs32<false>, KEPT>>(grid, st, c, 0); break;
+    case P_EMIT: launch_resident<k_pair32<ROWS, FLAT, PER, T, Pairs32<true>, KEPT>>(grid, st, c, 0); break;
+    case P_DIGEST: launch_resident<k_pair32<ROWS, FLAT, PER, T, Digest32, KEPT>>(grid, st, c, 0); break;
+    case P_FORCE_RHO0: launch_resident<k_pair32<ROWS, FLAT, PER, T, ForceRho032, KEPT>>(grid, st, c, 0); break;
+    case P_CONTINUITY: launch_resident<k_pair32<ROWS, FLAT, PER, T, Continuity32, KEPT>>(grid, st, c, 0); break;
     }
 }
 

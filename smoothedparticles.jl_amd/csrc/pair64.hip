@@ -646,7 +646,7 @@ __global__ __launch_bounds__(64, KEPT ? Op::WAVES_KEPT : Op::WAVES) void k_pair6
     const bool store_masks = ok && c.mask_mode == MASK_TEST_STORE;
     if ((load_masks && kept_ok) != KEPT) return;
     TileCursor tc;
-    tile_cursor_init(tc);
+    tile_cursor_init(c, ntiles, tc);
     // accepted pairs of all the wave's tiles, one atomic per wave
     unsigned npairs = 0;
     unsigned long long ntests = 0;
@@ -664,14 +664,14 @@ template <int ROWS, bool FLAT, bool PER, int T, bool KEPT>
 static void launch_tile_k(int op, const PairCtx& c, int grid, hipStream_t st)
 {
     switch (op) {
-    case P_DENSITY: k_pair64<ROWS, FLAT, PER, T, Density64<C_RHO>, KEPT><<<grid, 64, 0, st>>>(c); break;
-    case P_DENSITY_RHO0: k_pair64<ROWS, FLAT, PER, T, Density64<C_RHO0>, KEPT><<<grid, 64, 0, st>>>(c); break;
-    case P_FORCE: k_pair64<ROWS, FLAT, PER, T, Force64, KEPT><<<grid, 64, 0, st>>>(c); break;
-    case P_FORCE_RHO0: k_pair64<ROWS, FLAT, PER, T, ForceRho064, KEPT><<<grid, 64, 0, st>>>(c); break;
-    case P_CONTINUITY: k_pair64<ROWS, FLAT, PER, T, Continuity64, KEPT><<<grid, 64, 0, st>>>(c); break;
-    case P_COUNT: k_pair64<ROWS, FLAT, PER, T, Pairs64<false>, KEPT><<<grid, 64, 0, st>>>(c); break;
-    case P_EMIT: k_pair64<ROWS, FLAT, PER, T, Pairs64<true>, KEPT><<<grid, 64, 0, st>>>(c); break;
-    case P_DIGEST: k_pair64<ROWS, FLAT, PER, T, Digest64, KEPT><<<grid, 64, 0, st>>>(c); break;
+    case P_DENSITY: launch_resident<k_pair64<ROWS, FLAT, PER, T, Density64<C_RHO>, KEPT>>(grid, st, c); break;
+    case P_DENSITY_RHO0: launch_resident<k_pair64<ROWS, FLAT, PER, T, Density64<C_RHO0>, KEPT>>(grid, st, c); break;
+    case P_FORCE: launch_resident<k_pair64<ROWS, FLAT, PER, T, Force64, KEPT>>(grid, st, c); break;
+    case P_FORCE_RHO0: launch_resident<k_pair64<ROWS, FLAT, PER, T, ForceRho064, KEPT>>(grid, st, c); break;
+    case P_CONTINUITY: launch_resident<k_pair64<ROWS, FLAT, PER, T, Continuity64, KEPT>>(grid, st, c); break;
+    case P_COUNT: launch_resident<k_pair64<ROWS, FLAT, PER, T, Pairs64<false>, KEPT>>(grid, st, c); break;
+    case P_EMIT: launch_resident<k_pair64<ROWS, FLAT, PER, T, Pairs64<true>, KEPT>>(grid, st, c); break;
+    case P_DIGEST: launch_resident<k_pair64<ROWS, FLAT, PER, T, Digest64, KEPT>>(grid, st, c); break;
     }
 }
 

@@ -73,24 +73,41 @@ namespace sph {
 // distance and the direct form within ~1e-6 * h^2; the band is 10x wider.
 static constexpr double BAND = 1.0e-4;
 
+// The wave's copy of the counters.
+__device__ inline int counter_slot() { return (int)(blockIdx.x % CNT_COPIES) * CNT_STRIDE; }
+
 __device__ inline void count_pairs(const PairCtx& c, unsigned n)
 {
     // wave reduction of the per-lane counts, one atomic per wave
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) n += __shfl_xor(n, o);
-    if (__lane_id() == 0 && n) atomicAdd(c.pair_counter, (unsigned long long)n);
+    if (__lane_id() == 0 && n)
+        atomicAdd(c.pair_counter + counter_slot(), (unsigned long long)n);
 }
 
 // The wave's distance tests (the same value in every lane).
 __device__ inline void count_tests(const PairCtx& c, unsigned long long n)
 {
-    if (c.test_counter && __lane_id() == 0 && n) atomicAdd(c.test_counter, n);
+    if (c.test_counter && __lane_id() == 0 && n) atomicAdd(c.test_counter + counter_slot(), n);
 }
 
 // Tile queues.  The tile range [0, ntiles) is cut into NQUEUE contiguous
-// parts, one per queue head.  A wave starts on queue blockIdx % NQUEUE (the
-// XCD it runs on, so neighbouring tiles share that XCD's L2), takes qgrab
-// tiles per atomic, and when its queue is empty moves on to the next ones.
+// parts, one per queue head.  Block b belongs to queue b % NQUEUE (the XCD
+// it runs on, so neighbouring tiles share that XCD's L2).  The first tiles
+// of a queue are dealt out to its blocks without an atomic (block b takes
+// the (b / NQUEUE)-th share); the rest are taken qgrab at a time from the
+// queue head, and when its queue is empty a wave moves on to the others.
+// Only blocks that run at once may be dealt tiles -- a block that starts
+// when others leave would begin its share after all the rest -- so the grid
+// is what the chip holds (launch_resident; otherwise the force pass of a
+// 518k-particle collapse step takes 643 instead of 451 us).
+// An atomic on one head takes ~10.5 ns, one after the other: with every
+// tile behind an atomic, and every idle wave trying all heads, a pass took
+// 86 us however little it had to do (8192 waves on 8 heads; a 2D dam break of
+// 6514 particles: 13.6 -> 7.2 ms per 50 steps).  A queue whose tiles are all dealt
+// out is not touched.  (Reading another XCD's head before trying it spares
+// its last atomics but made the waves that help slower: the force pass of
+// the 5.75M-particle dam break took 3.25 instead of 3.06 ms.)
 // With one tile per grab the tiles in flight on an XCD are consecutive and
 // share their neighbour cells in the L2 (3D: 9.6 instead of 10.6 ms per
 // dam-break step); the short 2D tiles take four per grab, which spares
@@ -99,32 +116,47 @@ __device__ inline void count_tests(const PairCtx& c, unsigned long long n)
 // wave-uniform (readfirstlane), so the tile record, the system id and the
 // system's parameters are scalar loads held in SGPRs.
 struct TileCursor {
-    int q0, k, cur, end;
+    int k;         // queue in use, counted from the own one
+    int cur, end;  // tiles in hand
+    int deal;      // tiles each block is dealt
 };
 
-__device__ inline void tile_cursor_init(TileCursor& tc)
+__device__ inline int queue_lo(int ntiles, int q) { return (int)((long long)ntiles * q / NQUEUE); }
+
+// Tiles of queue q dealt out to its blocks.
+__device__ inline int queue_dealt(const TileCursor& tc, int q)
 {
-    tc.q0 = (int)(blockIdx.x % NQUEUE);
+    return (int)((gridDim.x + NQUEUE - 1 - q) / NQUEUE) * tc.deal;
+}
+
+__device__ inline void tile_cursor_init(const PairCtx& c, int ntiles, TileCursor& tc)
+{
+    // few tiles: one each, so that every block gets one before any gets two
+    tc.deal = (long long)gridDim.x * c.qgrab <= ntiles ? c.qgrab : 1;
     tc.k = 0;
-    tc.cur = tc.end = 0;
+    const int q = (int)(blockIdx.x % NQUEUE);
+    const int hi = queue_lo(ntiles, q + 1);
+    tc.cur = min(hi, queue_lo(ntiles, q) + (int)(blockIdx.x / NQUEUE) * tc.deal);
+    tc.end = min(hi, tc.cur + tc.deal);
 }
 
 __device__ inline int next_tile(const PairCtx& c, int ntiles, TileCursor& tc)
 {
     if (tc.cur < tc.end) return tc.cur++;
-    while (tc.k < NQUEUE) {
-        const int q = (tc.q0 + tc.k) % NQUEUE;
-        const int lo = (int)((long long)ntiles * q / NQUEUE);
-        const int hi = (int)((long long)ntiles * (q + 1) / NQUEUE);
+    for (; tc.k < NQUEUE; ++tc.k) {
+        const int q = (int)((blockIdx.x + tc.k) % NQUEUE);
+        const int dealt = queue_dealt(tc, q);
+        const int lo = queue_lo(ntiles, q) + dealt, hi = queue_lo(ntiles, q + 1);
+        if (lo >= hi) continue;
+        int* head = &c.queue[q * QSTRIDE];
         int start = 0;
-        if (__lane_id() == 0) start = atomicAdd(&c.queue[q * QSTRIDE], c.qgrab);
+        if (__lane_id() == 0) start = atomicAdd(head, c.qgrab);
         start = __builtin_amdgcn_readfirstlane(start);
         if (start < hi - lo) {
             tc.cur = lo + start;
             tc.end = min(hi, lo + start + c.qgrab);
             return tc.cur++;
         }
-        ++tc.k;
     }
     return ntiles;
 }
@@ -648,6 +680,31 @@ __device__ inline void digest_write(const PairCtx& c, int p, unsigned long long 
     const long long r = c.refidx[p];
     c.pair_out[2 * r] = (long long)n;
     c.pair_out[2 * r + 1] = (long long)h;
+}
+
+// -------------------------------------------------------------- launch --
+// Blocks of a kernel that the current device holds at once (one-wave
+// blocks, static LDS).
+inline int resident_blocks(const void* kernel)
+{
+    int dev = 0, cus = 0, per_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0) != hipSuccess ||
+        cus < 1 || per_cu < 1) {
+        (void)hipGetLastError();
+        return 256 * 8;
+    }
+    return cus * per_cu;
+}
+
+// Launch a tile kernel with the blocks it can use: no more than there are
+// tiles (grid) and no more than run at once.
+template <auto Kernel, class... Args>
+inline void launch_resident(int grid, hipStream_t st, Args... args)
+{
+    static const int fill = resident_blocks(reinterpret_cast<const void*>(Kernel));
+    Kernel<<<grid < fill ? grid : fill, 64, 0, st>>>(args...);
 }
 
 }  // namespace sph
