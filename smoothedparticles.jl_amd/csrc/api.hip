@@ -91,6 +91,7 @@ int make_geo(double h, const double* bmin, const double* bmax, int periodic, Geo
     g.h = h;
     g.inv_h = 1.0 / h;
     g.s_thr = sqrt_threshold(h);
+    g.tscale = std::ldexp(1.0, 9 - std::ilogb(h));
     for (int d = 0; d < 3; ++d) {
         if (!std::isfinite(bmin[d]) || !std::isfinite(bmax[d]) || bmin[d] > bmax[d])
             return fail(SPH_EINVAL, "invalid bounding box");

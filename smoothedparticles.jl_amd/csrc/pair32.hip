@@ -571,6 +571,15 @@ __device__ inline void tile32(const PairCtx& c, int tile, int out_col, bool load
         box.z0 = (float)(b.z0 - oz); box.z1 = (float)(b.z1 - oz);
         nr = build_cands<ROWS, PERIODIC>(d, c.cell_start, lc, L, total);
     }
+    // matrix-core test: centre of the box and the targets' operands
+    constexpr bool MFMA = !KEPT && T >= 32;
+    TestTile<MFMA ? T : 32> mt;
+    const float tsc = (float)d.g.tscale;
+    const float tcx = -0.5f * (box.x0 + box.x1) * tsc, tcy = -0.5f * (box.y0 + box.y1) * tsc;
+    const float tcz = FLAT ? 0.0f : -0.5f * (box.z0 + box.z1) * tsc;
+    if constexpr (MFMA)
+        test_targets<T>(mt, lane, fmaf(tg.x, tsc, tcx), fmaf(tg.y, tsc, tcy),
+                        FLAT ? 0.0f : fmaf(tg.z, tsc, tcz), (float)(d.g.h * d.g.tscale));
     __syncthreads();
     typename Op::Acc acc;
     Op::init(acc);
@@ -634,14 +643,18 @@ __device__ inline void tile32(const PairCtx& c, int tile, int out_col, bool load
             } else if (load_masks) {
                 if (s == 0 && act) word = c.masks[mbase + (long long)chunk * T + t];
             } else {
-                // 32-bit words, slots shifted in from the highest bit down
                 MaskT<T> m = 0, unsure = 0;
-#pragma unroll
-                for (int h = 0; h < (T + 31) / 32; ++h) {
+                if constexpr (MFMA) {
+                    const int sl = test_slot<T>(lane);
+                    const float4 a = lds.pos[rb + sl];
+                    test_chunk<T>(mt, fmaf(a.x, tsc, tcx), fmaf(a.y, tsc, tcy),
+                                  FLAT ? 0.0f : fmaf(a.z, tsc, tcz), sl >= fill - head, m, unsure);
+                } else {
+                    // slots shifted in from the highest bit down
                     unsigned min = 0, mout = 0;
 #pragma unroll 4
-                    for (int j = (T < 32 ? T : 32) - 1; j >= 0; --j) {
-                        const float4 a = lds.pos[rb + s + (64 / T) * (32 * h + j)];
+                    for (int j = T - 1; j >= 0; --j) {
+                        const float4 a = lds.pos[rb + s + (64 / T) * j];
                         const float q2 =
                             Op::STAGE_Q2 ? a.w : fmaf(a.z, a.z, fmaf(a.y, a.y, a.x * a.x));
                         float e = fmaf(mx, a.x, q2);
@@ -650,10 +663,9 @@ __device__ inline void tile32(const PairCtx& c, int tile, int out_col, bool load
                         min = shift_in_le(min, e, thr_in);
                         mout = shift_in_le(mout, e, thr_out);
                     }
-                    m |= (MaskT<T>)min << (32 * h);
-                    unsure |= (MaskT<T>)mout << (32 * h);
+                    m = min;
+                    unsure = mout & ~min;
                 }
-                unsure &= ~m;
                 if (!act) m = unsure = 0;
                 // the guard band: exact FP64 predicate of the reference (rare)
                 while (__any(unsure != 0)) {

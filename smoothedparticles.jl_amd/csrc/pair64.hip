@@ -490,6 +490,16 @@ __device__ inline void tile64(const PairCtx& c, int tile, bool load_masks, bool 
     if (!use_kept) box = ld_const(reinterpret_cast<const Box<double>*>(c.boxes) + tile);
     // (periodic systems need the ranges' image shifts in either case)
     if (!use_kept || PERIODIC) nr = build_cands<ROWS, PERIODIC>(d, c.cell_start, lc, L, total);
+    // matrix-core test: centre of the box and the targets' operands
+    constexpr bool MFMA = !KEPT && T >= 32;
+    TestTile<MFMA ? T : 32> mt;
+    const double tcx = 0.5 * (box.x0 + box.x1), tcy = 0.5 * (box.y0 + box.y1),
+                 tcz = 0.5 * (box.z0 + box.z1);
+    if constexpr (MFMA)
+        test_targets<T>(mt, lane, (float)((tg.x - tcx) * d.g.tscale),
+                        (float)((tg.y - tcy) * d.g.tscale),
+                        FLAT ? 0.0f : (float)((tg.z - tcz) * d.g.tscale),
+                        (float)(d.g.h * d.g.tscale));
     __syncthreads();
     typename Op::Acc acc;
     Op::init(acc);
@@ -550,14 +560,38 @@ __device__ inline void tile64(const PairCtx& c, int tile, bool load_masks, bool 
             } else if (load_masks) {
                 if (s == 0 && act) word = c.masks[mbase + (long long)chunk * T + t];
             } else {
-                // 32-bit words, slots shifted in from the highest bit down
                 MaskT<T> m = 0;
-#pragma unroll
-                for (int h = 0; h < (T + 31) / 32; ++h) {
+                if constexpr (MFMA) {
+                    MaskT<T> unsure = 0;
+                    const int sl = test_slot<T>(lane);
+                    const double2 qxy = lds.xy[rb + sl];
+                    const double qz = FLAT ? 0.0 : lds_z(lds, rb + sl);
+                    test_chunk<T>(mt, (float)((qxy.x - tcx) * d.g.tscale),
+                                  (float)((qxy.y - tcy) * d.g.tscale),
+                                  FLAT ? 0.0f : (float)((qz - tcz) * d.g.tscale),
+                                  sl >= fill - head, m, unsure);
+                    // near the threshold: the exact predicate of the reference
+                    while (__any(unsure != 0)) {
+                        if (unsure) {
+                            const int j = lowest_bit<T>(unsure);
+                            unsure &= unsure - 1;
+                            const int jj = rb + s + (64 / T) * j;
+                            const double2 xy = lds.xy[jj];
+                            const double dx = tg.x - xy.x, dy = tg.y - xy.y;
+                            double ss = dx * dx + dy * dy;
+                            if (!FLAT) {
+                                const double dz = tg.z - lds_z(lds, jj);
+                                ss = ss + dz * dz;
+                            }
+                            if (ss <= s_thr) m |= MaskT<T>(1) << j;
+                        }
+                    }
+                } else {
+                    // slots shifted in from the highest bit down
                     unsigned mh = 0;
 #pragma unroll 4
-                    for (int j = (T < 32 ? T : 32) - 1; j >= 0; --j) {
-                        const int jj = rb + s + (64 / T) * (32 * h + j);
+                    for (int j = T - 1; j >= 0; --j) {
+                        const int jj = rb + s + (64 / T) * j;
                         const double2 xy = lds.xy[jj];
                         const double dx = tg.x - xy.x, dy = tg.y - xy.y;
                         double ss = dx * dx + dy * dy;
@@ -567,7 +601,7 @@ __device__ inline void tile64(const PairCtx& c, int tile, bool load_masks, bool 
                         }
                         mh = shift_in_le(mh, ss, s_thr);
                     }
-                    m |= (MaskT<T>)mh << (32 * h);
+                    m = mh;
                 }
                 if (!act) m = 0;
                 drop_self<ROWS, PERIODIC, T>(L, nself, head, t, s, m);

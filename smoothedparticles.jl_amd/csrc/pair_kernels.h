@@ -200,6 +200,188 @@ __device__ inline int lowest_bit(MaskT<T> m)
     else return __ffs(m) - 1;
 }
 
+// ------------------------------------------------- matrix-core candidate test --
+// The test of a chunk's 64 slots against the tile's targets, for T = 64 and
+// 32, as a product on the matrix cores: with the target p and the candidate
+// q relative to the centre of the targets' box,
+//     D = |q|^2 - 2 p.q + (|p|^2 - h^2)
+// is a sum of 16 products of 16-bit floats once every coordinate, |q|^2 and
+// |p|^2 - h^2 are split into a high and a low half (11 + 11 bits): four
+// products per axis, two for |q|^2, two for |p|^2 - h^2.  That is one
+// v_mfma_f32_32x32x16_f16 per 32 x 32 block (32 cycles), and the sign of D is
+// the answer: one v_alignbit shifts it into the lane's mask.  Per chunk and
+// lane that is ~150 vector instructions where three FMAs and two compares
+// with carry per test took 448, and no LDS read per test.
+//
+// D is only a filter.  Coordinates are scaled by a power of two to
+// 512 <= h < 1024, so no half overflows or loses bits to underflow; the
+// halves keep 2^-21 of a value and the sum of 16 products in FP32 loses at
+// most 16 * 2^-23 of its largest partial sum (8 h^2): together below 2e-5 h^2.
+// A pair with |D| below TEST_BAND h^2 (twice that) is settled by the exact
+// FP64 predicate, as in the FP32 test; found by a minimum over the lane's 16
+// values per block, and looked for bit by bit only in blocks that hold one
+// (about one in twenty).  So the masks are the reference's sets, bit for bit
+// what they were.
+//
+// Layout: acc[i] of lane l holds row 8 (i / 4) + 4 (l / 32) + i % 4 (the
+// candidate, operand A) and column l % 32 (the target, operand B); an operand
+// lane l holds elements 8 (l / 32) ... + 7 of row l % 32.  Each lane splits
+// one slot (and, once per tile, one target) into eight packed registers, the
+// first four for l < 32; v_permlane32_swap of register i with i + 4 gives
+// both 32-row operands.  Lane l takes slot test_slot(l), so that the bits
+// come out in the order of the masks.
+//
+// Density pass of the 5.75M-particle dam break: 3.79 -> 3.34 ms (mixed);
+// of a 1.5M-particle one in FP64: 2.86 -> 2.20 ms.  T = 16 and 8 would leave
+// half or more of the columns empty and keep the vector test.
+static constexpr double TEST_BAND = 4.0e-5;
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float acc16_t __attribute__((ext_vector_type(16)));
+typedef __fp16 half2_t __attribute__((ext_vector_type(2)));
+
+// (a, b) as packed 16-bit floats, rounded towards zero, and what that left.
+__device__ inline unsigned split_pair(float a, float b, unsigned& rest)
+{
+    const half2_t h = __builtin_amdgcn_cvt_pkrtz(a, b);
+    const half2_t r = __builtin_amdgcn_cvt_pkrtz(a - (float)h[0], b - (float)h[1]);
+    rest = __builtin_bit_cast(unsigned, r);
+    return __builtin_bit_cast(unsigned, h);
+}
+
+__device__ inline half8_t as_half8(const unsigned* r)
+{
+    struct R {
+        unsigned v[4];
+    } t = {{r[0], r[1], r[2], r[3]}};
+    return __builtin_bit_cast(half8_t, t);
+}
+
+static constexpr unsigned HALF2_256 = 0x5c005c00u;  // (256, 256)
+
+// Slot of the chunk whose candidate lane l holds.
+template <int T>
+__device__ inline int test_slot(int l)
+{
+    const int hf = (l >> 2) & 1, b = (l >> 5) * 16 + ((l >> 3) & 3) * 4 + (l & 3);
+    return T == 64 ? hf * 32 + b : hf + 2 * b;
+}
+
+template <int T>
+struct TestTile {
+    half8_t p[T / 32];  // targets, 32 rows each
+    float band;
+};
+
+// x, y, z: the lane's target (lane % T), relative to the centre and scaled;
+// hs: h scaled.
+template <int T>
+__device__ inline void test_targets(TestTile<T>& tt, int lane, float x, float y, float z, float hs)
+{
+    const float w = (fmaf(z, z, fmaf(y, y, x * x)) - hs * hs) * (1.0f / 256.0f);
+    unsigned r[8], zw, zwl;
+    r[0] = split_pair(-2.0f * x, -2.0f * y, r[1]);
+    zw = split_pair(-2.0f * z, w, zwl);
+    r[2] = r[0];
+    r[3] = r[1];
+    r[4] = (zw & 0xffffu) | (HALF2_256 & 0xffff0000u);  // (z, 256)
+    r[5] = r[4];
+    r[6] = (zwl & 0xffffu) | (zwl << 16);               // (z low, z low)
+    r[7] = (zw >> 16) | (zwl & 0xffff0000u);            // (w, w low)
+    if constexpr (T == 64) {
+        unsigned a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const auto s = __builtin_amdgcn_permlane32_swap(r[i], r[i + 4], false, false);
+            a[i] = s[0];
+            b[i] = s[1];
+        }
+        tt.p[0] = as_half8(a);
+        tt.p[1] = as_half8(b);
+    } else {
+        unsigned a[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = lane < 32 ? r[i] : r[i + 4];
+        tt.p[0] = as_half8(a);
+    }
+    tt.band = (float)TEST_BAND * hs * hs;
+}
+
+// x, y, z: the candidate in slot test_slot(lane), relative to the centre and
+// scaled; pad: the slot is past the end of the list.  m: the lane's mask of
+// accepted slots (of target lane % T; bit j of slice s is slot s + (64/T) j),
+// unsure: those the exact test has to settle.
+template <int T>
+__device__ inline void test_chunk(const TestTile<T>& tt, float x, float y, float z, bool pad,
+                                  MaskT<T>& m, MaskT<T>& unsure)
+{
+    x = pad ? 0.0f : x;
+    y = pad ? 0.0f : y;
+    z = pad ? 0.0f : z;
+    const float q2 = pad ? 60000.0f : fmaf(z, z, fmaf(y, y, x * x)) * (1.0f / 256.0f);
+    unsigned r[8];
+    r[0] = split_pair(x, y, r[2]);
+    r[1] = r[0];
+    r[3] = r[2];
+    r[4] = split_pair(z, q2, r[5]);
+    r[6] = (r[4] & 0xffffu) | (r[5] << 16);  // (z, z low)
+    r[7] = HALF2_256;
+    half8_t q[2];
+    {
+        unsigned a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const auto s = __builtin_amdgcn_permlane32_swap(r[i], r[i + 4], false, false);
+            a[i] = s[0];
+            b[i] = s[1];
+        }
+        q[0] = as_half8(a);
+        q[1] = as_half8(b);
+    }
+    unsigned mm[T / 32], uu[T / 32];
+#pragma unroll
+    for (int k = 0; k < T / 32; ++k) mm[k] = uu[k] = 0;
+    bool any = false;
+#pragma unroll
+    for (int cb = 1; cb >= 0; --cb)
+#pragma unroll
+        for (int k = 0; k < T / 32; ++k) {
+            acc16_t d = {};
+            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(q[cb], tt.p[k], d, 0, 0, 0);
+            float near = fabsf(d[0]);
+#pragma unroll
+            for (int i = 15; i >= 0; --i)
+                mm[k] = __builtin_amdgcn_alignbit(mm[k], __float_as_uint(d[i]), 31);
+#pragma unroll
+            for (int i = 1; i < 15; i += 2) near = fminf(fminf(fabsf(d[i]), fabsf(d[i + 1])), near);
+            near = fminf(fabsf(d[15]), near);
+            // one block's 16 results at a time: without this the compiler
+            // keeps the four blocks' 64 live and spills (+70 registers)
+            asm volatile("" : "+v"(mm[k]), "+v"(near));
+            uu[k] <<= 16;
+            if (__any(near < tt.band)) {
+                any = true;
+                unsigned u = 0;
+#pragma unroll
+                for (int i = 15; i >= 0; --i) u = u * 2 + (fabsf(d[i]) < tt.band ? 1u : 0u);
+                uu[k] |= u;
+            }
+        }
+    if constexpr (T == 64) {
+        const auto s = __builtin_amdgcn_permlane32_swap(mm[0], mm[1], false, false);
+        m = (MaskT<T>)s[0] | ((MaskT<T>)s[1] << 32);
+        unsure = 0;
+        if (any) {
+            const auto v = __builtin_amdgcn_permlane32_swap(uu[0], uu[1], false, false);
+            unsure = (MaskT<T>)v[0] | ((MaskT<T>)v[1] << 32);
+        }
+    } else {
+        m = mm[0];
+        unsure = uu[0];
+    }
+    m &= ~unsure;
+}
+
 // ------------------------------------------------------------ candidates --
 // The candidate ranges of a tile: its cell's stencil rows, concatenated.
 // pref[i] candidates precede range i; a chunk's slot l holds candidate

@@ -66,6 +66,7 @@ struct Geo {
     int pad;
     double box[3];   // periodic box lengths (bmax - bmin)
     double cell[3];  // periodic cell lengths box / L (>= h)
+    double tscale;   // power of two with 512 <= h * tscale < 1024 (candidate test)
 };
 
 // Parameters of the pair and unary kernels (derived from sph_params).
