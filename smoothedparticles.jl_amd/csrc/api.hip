@@ -19,7 +19,7 @@
 using namespace sph;
 
 namespace sph {
-void enqueue_build(sph_system* s, unsigned skip_cols = 0);
+void enqueue_build(sph_system* s, unsigned skip_cols = 0, int skip_a = 0);
 void enqueue_tiles(sph_system* s);
 void enqueue_unary(sph_system* s, int op, double* prho2);
 void enqueue_prho2(sph_system* s);
@@ -48,6 +48,7 @@ void enqueue_lattice_write(sph_system* s, const LatticeGeo& g, const sph_lattice
 void enqueue_fill_int(sph_system* s, int* p, int v, long long n);
 void enqueue_remap_sys(sph_system* s, const int* map_dev);
 long long scan_partials_needed(long long n);
+long long scan_state_needed(long long cells);
 long long reduce_partials_needed(long long n);
 void reset_queue(sph_system* s);
 }  // namespace sph
@@ -199,9 +200,8 @@ void free_particle_arrays(sph_system* s)
         dfree(s, s->icols[b], NICOL * cap);
     }
     dfree(s, s->slot, cap); dfree(s, s->tmp_idx, cap); dfree(s, s->tmp_key, cap);
-    dfree(s, s->tmp_ref, cap); dfree(s, s->perm, cap); dfree(s, s->inv, cap);
+    dfree(s, s->tmp_ref, cap); dfree(s, s->inv, cap);
     dfree(s, s->tiles, s->tile_cap); dfree(s, s->kept_n, s->tile_cap);
-    dfree(s, s->boxes, 6 * s->tile_cap);
     dfree(s, s->prho2, cap); dfree(s, s->stage, 9 * cap);
     dfree(s, s->red_part, s->red_part_n);
 }
@@ -252,9 +252,9 @@ int ensure_capacity(sph_system* s, long long need)
     s->red_part_n = 3 * reduce_partials_needed(ncap);
     if ((rc = dalloc(s, &s->slot, ncap)) || (rc = dalloc(s, &s->tmp_idx, ncap)) ||
         (rc = dalloc(s, &s->tmp_key, ncap)) || (rc = dalloc(s, &s->tmp_ref, ncap)) ||
-        (rc = dalloc(s, &s->perm, ncap)) || (rc = dalloc(s, &s->inv, ncap)) ||
+        (rc = dalloc(s, &s->inv, ncap)) ||
         (rc = dalloc(s, &s->tiles, s->tile_cap)) || (rc = dalloc(s, &s->kept_n, s->tile_cap)) ||
-        (rc = dalloc(s, &s->boxes, 6 * s->tile_cap)) || (rc = dalloc(s, &s->prho2, ncap)) ||
+        (rc = dalloc(s, &s->prho2, ncap)) ||
         (rc = dalloc(s, &s->stage, 9 * ncap)) || (rc = dalloc(s, &s->red_part, s->red_part_n)))
         return rc;
     return 0;
@@ -263,10 +263,8 @@ int ensure_capacity(sph_system* s, long long need)
 void free_cell_arrays(sph_system* s)
 {
     const long long c = s->cells_cap;
-    dfree(s, s->cnt, c); dfree(s, s->cell_start, c + 1); dfree(s, s->tile_start, c + 1);
-    dfree(s, s->cell_chunks, c); dfree(s, s->mask_start, c + 1); dfree(s, s->cell_sys, c);
-    dfree(s, s->cell_order, c);
-    dfree(s, s->scan_part, s->scan_part_n); dfree(s, s->scan_part64, s->scan_part_n);
+    dfree(s, s->cnt, c); dfree(s, s->cell_start, c + 1); dfree(s, s->cell_sys, c);
+    dfree(s, s->scan_state, s->scan_state_n);
 }
 
 // Per-cell arrays for `buckets` buckets (the cells of every system, one
@@ -279,23 +277,21 @@ int ensure_cells(sph_system* s, long long buckets)
     if (ncap >= (1ll << 31) - 64) return fail(SPH_EINVAL, "too many cells in the batch");
     free_cell_arrays(s);
     s->cells_cap = ncap;
-    s->scan_part_n = scan_partials_needed(ncap + 2);
+    s->scan_state_n = scan_state_needed(ncap);
     int rc;
     if ((rc = dalloc(s, &s->cnt, ncap)) || (rc = dalloc(s, &s->cell_start, ncap + 1)) ||
-        (rc = dalloc(s, &s->tile_start, ncap + 1)) || (rc = dalloc(s, &s->cell_chunks, ncap)) ||
-        (rc = dalloc(s, &s->mask_start, ncap + 1)) || (rc = dalloc(s, &s->cell_sys, ncap)) ||
-        (rc = dalloc(s, &s->cell_order, ncap)) || (rc = dalloc(s, &s->scan_part, s->scan_part_n)) ||
-        (rc = dalloc(s, &s->scan_part64, s->scan_part_n))) {
+        (rc = dalloc(s, &s->cell_sys, ncap)) ||
+        (rc = dalloc(s, &s->scan_state, s->scan_state_n))) {
         s->cells_cap = 0;
         return rc;
     }
+    // a build finds the counts cleared and leaves them so
+    HIPC(hipMemsetAsync(s->cnt, 0, sizeof(unsigned) * ncap, s->stream));
     if (s->cap > 0) {  // the tile bound grows with the cell count
         dfree(s, s->tiles, s->tile_cap);
         dfree(s, s->kept_n, s->tile_cap);
-        dfree(s, s->boxes, 6 * s->tile_cap);
         s->tile_cap = tile_bound(s);
-        if ((rc = dalloc(s, &s->tiles, s->tile_cap)) || (rc = dalloc(s, &s->kept_n, s->tile_cap)) ||
-            (rc = dalloc(s, &s->boxes, 6 * s->tile_cap)))
+        if ((rc = dalloc(s, &s->tiles, s->tile_cap)) || (rc = dalloc(s, &s->kept_n, s->tile_cap)))
             return rc;
     }
     for (int i = 0; i < nsys(s); ++i)
@@ -430,7 +426,6 @@ PairCtx make_ctx(sph_system* s)
     c.kept = s->use_kept ? s->kept : nullptr;
     c.kept_rg = s->kept_rg;
     c.kept_n = s->kept_n;
-    c.boxes = s->boxes;
     c.mask_mode = MASK_TEST;
     c.masks_mixed = s->precision == SPH_MIXED;
     return c;
@@ -511,9 +506,11 @@ int pair_grid(long long ntiles)
     return (int)std::max<long long>(g, 1);
 }
 
+// queue_set: the set of tile-queue heads to use, as the last build cleared it
+// (each at most once per build), or -1 to clear set 0 first.
 int run_pair(sph_system* s, int op, int self, int overwrite, unsigned long long* counter,
              long long ntiles, int prof_kernel, int mask_mode, int only_flagged = 0,
-             unsigned long long* tests = nullptr)
+             unsigned long long* tests = nullptr, int queue_set = -1)
 {
     PairCtx c = make_ctx(s);
     c.self = self;
@@ -524,7 +521,8 @@ int run_pair(sph_system* s, int op, int self, int overwrite, unsigned long long*
     c.only_flagged = only_flagged;
     hipEvent_t ev[2];
     prof_begin(s, ev);
-    reset_queue(s);
+    if (queue_set < 0) reset_queue(s);
+    else c.queue += queue_set * NQUEUE * QSTRIDE;
     launch_pair(op, s->precision, s->rows, s->flat, s->periodic, c, pair_grid(ntiles), s->stream);
     prof_end(s, prof_kernel, ev);
     HIPC(hipGetLastError());
@@ -575,7 +573,7 @@ int new_handle(int precision, sph_system** out)
         rc = fail(SPH_EHIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
     }
     if (!rc && !(rc = dalloc(s, &s->meta, META_SLOTS)) && !(rc = dalloc(s, &s->pair_counter, CNT_SLOTS)) &&
-        !(rc = dalloc(s, &s->queue, NQUEUE * QSTRIDE)) &&
+        !(rc = dalloc(s, &s->queue, NQUEUE_SETS * NQUEUE * QSTRIDE)) &&
         !(rc = dalloc(s, &s->red_out, 4)) && !(rc = dalloc(s, &s->mask_total, 1))) {
         e = hipHostMalloc((void**)&s->meta_host, sizeof(int) * META_SLOTS, hipHostMallocDefault);
         if (e != hipSuccess) s->meta_host = nullptr;
@@ -613,7 +611,7 @@ int destroy(sph_system* s)
     free_particle_arrays(s);
     free_cell_arrays(s);
     dfree(s, s->meta, META_SLOTS); dfree(s, s->pair_counter, CNT_SLOTS); dfree(s, s->red_out, 4);
-    dfree(s, s->queue, NQUEUE * QSTRIDE);
+    dfree(s, s->queue, NQUEUE_SETS * NQUEUE * QSTRIDE);
     dfree(s, s->masks, s->mask_cap); dfree(s, s->mask_total, 1);
     dfree(s, s->kept, s->kept_cap); dfree(s, s->kept_rg, s->kept_cap);
     dfree(s, s->sysd, s->sysd_cap); dfree(s, s->sys_cnt, SYSCNT * s->sys_cnt_cap);
@@ -827,7 +825,7 @@ int cd_step(sph_system* s, long long tiles_bound)
     enqueue_build(s);
     prof_end(s, SPH_KERNEL_BUILD, ev);
     if ((rc = run_pair(s, P_CONTINUITY, 0, 0, s->pair_counter, tiles_bound, SPH_KERNEL_DENSITY,
-                       MASK_TEST, 0, s->pair_counter + 2)))
+                       MASK_TEST, 0, s->pair_counter + 2, 0)))
         return rc;
     prof_begin(s, ev);
     enqueue_unary(s, SPH_OP_FIND_PRESSURE_CONTINUITY, nullptr);
@@ -838,7 +836,7 @@ int cd_step(sph_system* s, long long tiles_bound)
     prof_end(s, SPH_KERNEL_BUILD, ev);
     enqueue_prho2(s);  // the build permuted the particles
     if ((rc = run_pair(s, P_FORCE, 0, 0, s->pair_counter + 1, tiles_bound, SPH_KERNEL_FORCE,
-                       MASK_TEST)))
+                       MASK_TEST, 0, nullptr, 1)))
         return rc;
     prof_begin(s, ev);
     enqueue_cd_unary(s, CD_KICK);
@@ -856,17 +854,18 @@ int ds_step(sph_system* s, int eos, long long tiles_bound)
     prof_begin(s, ev);
     // the density pass overwrites rho of every particle in a cell and the
     // EOS then P of every particle, before anything reads them: the build
-    // need not carry the two columns over
-    enqueue_build(s, (1u << C_RHO) | (1u << C_P));
+    // need not carry the two columns over, nor the acceleration of the fluid,
+    // which the force pass overwrites
+    enqueue_build(s, (1u << C_RHO) | (1u << C_P), 1);
     prof_end(s, SPH_KERNEL_BUILD, ev);
     if ((rc = run_pair(s, P_DENSITY, 1, 1, s->pair_counter, tiles_bound, SPH_KERNEL_DENSITY,
-                       MASK_TEST_STORE, 0, s->pair_counter + 2)))
+                       MASK_TEST_STORE, 0, s->pair_counter + 2, 0)))
         return rc;
     prof_begin(s, ev);
     enqueue_unary(s, eos, s->prho2);
     prof_end(s, SPH_KERNEL_UNARY, ev);
     if ((rc = run_pair(s, P_FORCE, 0, 1, s->pair_counter + 1, tiles_bound, SPH_KERNEL_FORCE,
-                       MASK_LOAD)))
+                       MASK_LOAD, 0, nullptr, 1)))
         return rc;
     prof_begin(s, ev);
     enqueue_kick_drift(s);

@@ -1,49 +1,48 @@
 // Cell-list builder: the device form of create_cell_list! (src/core.jl:51-90)
 // for every system of a batch at once.
 //
-// Stages, all on the handle's stream, no host round trip:
-//   1. k_keys     per particle: FP64 find_key (src/structs.jl:97-106) and the
-//                 inclusive bounding-box test (src/geometry.jl:24-30); a
-//                 particle outside goes to its system's removal bucket.
-//                 Periodic systems wrap positions into the box instead.
-//                 Global key = the system's cell_base + local key.  Per-bucket
-//                 counts by wave-aggregated atomics (one atomic per distinct
-//                 key in a wave; the input is the previous sorted order, so a
-//                 wave usually touches one or two cells).
-//   2. scan       exclusive prefix sum of the counts -> cell_start
-//   3. k_scatter  bucket every particle
-//   4. k_rank     order each bucket by descending reference index, the order
-//                 add_index! keeps (src/core.jl:26-41); deterministic
-//                 whatever order the atomics handed out (the bucket of
-//                 retired systems keeps its scatter order, never used)
-//   5. k_gather   permute every column into the new order
-//   6. removal    each system's removal bucket holds its removed particles in
-//                 descending reference index; the reference's swap-with-end
-//                 renumbering (src/core.jl:72-81) is replayed per system
-//   7. tiles      a scan of ceil(count/T) per cell, the 64-candidate chunks a
-//                 target of each cell walks, a scan of pair-mask words, and
-//                 the tile table of the pair kernels
+// Five kernels, all on the handle's stream, no host round trip:
+//   1. k_keys        per particle: FP64 find_key (src/structs.jl:97-106) and
+//                    the inclusive bounding-box test (src/geometry.jl:24-30);
+//                    a particle outside goes to its system's removal bucket.
+//                    Periodic systems wrap positions into the box instead.
+//                    Global key = the system's cell_base + local key.
+//                    Per-bucket counts by wave-aggregated atomics (one atomic
+//                    per distinct key in a wave; the input is the previous
+//                    sorted order, so a wave usually touches one or two cells)
+//   2. k_scan_counts exclusive prefix sum of the counts -> cell_start
+//   3. k_scatter     bucket every particle
+//   4. k_place       order each bucket by descending reference index, the
+//                    order add_index! keeps (src/core.jl:26-41) -- deterministic
+//                    whatever order the atomics handed out; the bucket of
+//                    retired systems keeps its scatter order, never used --
+//                    and move every column into the new order
+//   5. k_tile_table  per cell ceil(count/T) tiles and the 64-candidate chunks
+//                    a target walks, one scan of both, the tile table of the
+//                    pair kernels.  Also the removal: each system's removal
+//                    bucket holds its removed particles in descending
+//                    reference index, and the reference's swap-with-end
+//                    renumbering (src/core.jl:72-81) is replayed per system
 //
 // This is a counting sort on the global cell key (one radix digit) followed
 // by an in-bucket rank.
+//
+// A small system's build is bound by its launches: with 19 kernels (three for
+// each of three scans, of 5 + 3 + 12 us whatever their length) it took about
+// 100 us, 30 us with these five; the 5.75M-particle dam break's took 560 us,
+// 390 us now (no permutation written and read back, the fluid's acceleration
+// left out, no pass for the tiles' boxes).
 #include "scan_kernels.h"
 #include "sph_internal.h"
 
 namespace sph {
 
 
-__global__ void k_fill_u32(unsigned* p, unsigned v, long long n)
-{
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
 // ---------------------------------------------------------------- prepare --
 // Per-system reference-index base of the inverse map and the count at the
-// start of the build.
-// One block of 256 threads; systems in rounds of 256, an exclusive scan of
-// the counts per round.
-__global__ __launch_bounds__(256) void k_sys_prep(int nsys, int* sc, int* meta)
+// start of the build.  One block of 256 threads; systems in rounds of 256, an
+// exclusive scan of the counts per round.
+__device__ inline void sys_prep(int nsys, int* sc, int* meta)
 {
     __shared__ int part[4];
     int carry = 0;
@@ -119,12 +118,16 @@ __device__ inline int key_of(const SysDesc& d, int s, int nsys, int cells_total,
 
 __global__ __launch_bounds__(256) void k_keys(const SysDesc* __restrict__ sysd, int nsys,
                                               int cells_total, double* x, double* y, double* z,
-                                              const int* __restrict__ sysid, const int* meta,
+                                              const int* __restrict__ sysid, int* meta,
                                               int* __restrict__ key, int* __restrict__ slot,
-                                              unsigned* __restrict__ cnt)
+                                              unsigned* __restrict__ cnt, int* sc,
+                                              unsigned long long* stat, int nstat)
 {
     const int n = meta[META_N];
     const int i = blockIdx.x * 256 + threadIdx.x;
+    // the scans of this build start from cleared state words
+    for (int j = i; j < nstat; j += gridDim.x * 256) stat[j] = 0ull;
+    if (blockIdx.x == 0) sys_prep(nsys, sc, meta);
     const int s = i < n ? sysid[i] : 0;
     // a wave of one system reads its descriptor once, through the scalar
     // cache (the usual case: systems are contiguous)
@@ -155,44 +158,52 @@ __global__ __launch_bounds__(256) void k_keys(const SysDesc* __restrict__ sysd, 
 }
 
 // ------------------------------------------------------------------ scan --
-// (kernels in scan_kernels.h)
-struct SrcCount {
-    using V = unsigned;
-    const unsigned* c;
-    __device__ V operator()(int i) const { return c[i]; }
-};
-// Tiles of the cell at brick rank i: ceil(count / T).
-struct SrcTiles {
-    using V = unsigned;
-    const int* cs;
-    const int* order;
-    int ncells;
-    int T;
-    __device__ V operator()(int i) const
-    {
-        if (i >= ncells) return 0u;
-        const int c = order[i];
-        const int n = cs[c + 1] - cs[c];
-        return (unsigned)((n + T - 1) / T);
-    }
-};
-// Mask words of the cell at brick rank i: tiles * chunks per target * T.
-struct SrcMaskWords {
-    using V = unsigned long long;
-    const int* tile_start;
-    const int* chunks;
-    const int* order;
-    int ncells;
-    int T;
-    __device__ V operator()(int i) const
-    {
-        if (i >= ncells) return 0ull;
-        const long long nt = tile_start[i + 1] - tile_start[i];
-        return (V)(nt * chunks[order[i]] * T);
-    }
-};
-
 long long scan_partials_needed(long long n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 1; }
+
+// Exclusive prefix sum of the bucket counts into start[0 .. n], in one
+// launch (chained blocks, scan_kernels.h).  The counts are zeroed behind the
+// read: the next build finds them cleared.
+static constexpr int CSCAN_TILE = 256 * 8;
+
+__global__ __launch_bounds__(256) void k_scan_counts(unsigned* cnt, int n, int* start,
+                                                     unsigned long long* stat,
+                                                     unsigned long long* ticket)
+{
+    __shared__ unsigned long long prefix;
+    const int b = chain_ticket(ticket);
+    const int base = b * CSCAN_TILE + (int)threadIdx.x * 8;
+    unsigned v[8];
+    unsigned sum = 0;
+    if (base + 8 <= n) {
+        const uint4 lo = *reinterpret_cast<const uint4*>(cnt + base);
+        const uint4 hi = *reinterpret_cast<const uint4*>(cnt + base + 4);
+        v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w;
+        v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+        *reinterpret_cast<uint4*>(cnt + base) = make_uint4(0u, 0u, 0u, 0u);
+        *reinterpret_cast<uint4*>(cnt + base + 4) = make_uint4(0u, 0u, 0u, 0u);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            v[k] = base + k < n ? cnt[base + k] : 0u;
+            if (base + k < n) cnt[base + k] = 0u;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) sum += v[k];
+    unsigned total;
+    unsigned run = block_incl_scan(sum, total) - sum;
+    if (threadIdx.x < 64) {
+        const unsigned long long p = chain_prefix(stat, b, total);
+        if (threadIdx.x == 0) prefix = p;
+    }
+    __syncthreads();
+    run += (unsigned)prefix;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (base + k <= n) start[base + k] = (int)run;
+        run += v[k];
+    }
+}
 
 // -------------------------------------------------- scatter, rank, gather --
 __global__ __launch_bounds__(256) void k_scatter(const int* meta, const int* __restrict__ key,
@@ -211,6 +222,62 @@ __global__ __launch_bounds__(256) void k_scatter(const int* meta, const int* __r
     tmp_ref[pos] = ref[i];
 }
 
+// Totals of the build, per system and overall (one block of 256 threads).
+__device__ inline void finalize(const SysDesc* __restrict__ sysd, int nsys, int cells_total,
+                                int* sc, int* meta, const int* cell_start)
+{
+    if (threadIdx.x == 0) {
+        const int na = cell_start[cells_total];
+        meta[META_NREM] = meta[META_NTOT] - na;
+        meta[META_N] = na;
+        meta[META_NCELLS] = 0;
+    }
+    for (int s = threadIdx.x; s < nsys; s += 256) {
+        const SysDesc& d = sysd[s];
+        const int off = cell_start[d.cell_base];
+        const int end = cell_start[d.cell_base + d.g.key_max];
+        sc[SYSCNT * s + SC_OFF] = off;
+        sc[SYSCNT * s + SC_N] = d.live ? end - off : 0;
+        sc[SYSCNT * s + SC_NREM] = cell_start[cells_total + s + 1] - cell_start[cells_total + s];
+    }
+}
+
+// What k_place moves: the columns and where they go.
+struct Move {
+    const double* src;
+    double* dst;
+    const int* isrc;
+    int* idst;
+    long long cap;
+    unsigned skip;     // columns (bit C_*) left out
+    int skip_a;        // leave out the acceleration of fluid particles
+    const int* sc;     // per-system counters (reference-index base)
+    int* inv;
+};
+
+// Particle j of the old order, with reference index r, to slot k of the new
+// one; with removals in this build, inv maps (system reference base +
+// reference index) to the slot.
+__device__ inline void move_particle(const Move& mv, int j, int key, int r, int k, bool removals)
+{
+#pragma unroll
+    for (int f = 0; f < NCOL; ++f)
+        if (f != C_AX && f != C_AY && f != C_AZ && f != C_TYPE && !((mv.skip >> f) & 1u))
+            mv.dst[f * mv.cap + k] = mv.src[f * mv.cap + j];
+    const double type = mv.src[C_TYPE * mv.cap + j];
+    mv.dst[C_TYPE * mv.cap + k] = type;
+    if (!mv.skip_a || type != 0.0) {
+        mv.dst[C_AX * mv.cap + k] = mv.src[C_AX * mv.cap + j];
+        mv.dst[C_AY * mv.cap + k] = mv.src[C_AY * mv.cap + j];
+        mv.dst[C_AZ * mv.cap + k] = mv.src[C_AZ * mv.cap + j];
+    }
+    const int s = mv.isrc[I_SYS * mv.cap + j];
+    mv.idst[I_REF * mv.cap + k] = r;
+    mv.idst[I_KEY * mv.cap + k] = key;
+    mv.idst[I_SYS * mv.cap + k] = s;
+    if (removals) mv.inv[mv.sc[SYSCNT * s + SC_REFBASE] + r] = k;
+}
+
 // Rank of each particle in its bucket: the number of bucket members with a
 // larger reference index (ties -- particles of different retired systems --
 // by scatter position), so the ranks are a permutation of the bucket.
@@ -223,20 +290,18 @@ __global__ __launch_bounds__(256) void k_scatter(const int* meta, const int* __r
 //     to hundreds of particles) are staged through LDS when they fit in
 //     RANK_SPAN entries, and each thread counts against its bucket there;
 //   - else each thread scans its bucket in global memory.
+// The thread then moves its particle: it reads near the old slot and writes
+// inside its bucket, so both sides of the permutation stay within a few cache
+// lines of its neighbours' (the 5.75M-particle dam break: rank and gather
+// apart 61 + 232 us, together 274 us).
 static constexpr int RANK_LDS_MIN = 512;
 static constexpr int RANK_SPAN = 2048;
 
-__global__ __launch_bounds__(256) void k_rank(const int* meta, const int* __restrict__ cell_start,
-                                              const int* __restrict__ tmp_idx,
-                                              const int* __restrict__ tmp_key,
-                                              const int* __restrict__ tmp_ref, int* perm,
-                                              int dead_key)
+__device__ inline int rank_in_bucket(int b0, int n, const int* __restrict__ cell_start,
+                                     const int* __restrict__ tmp_key,
+                                     const int* __restrict__ tmp_ref, int dead_key, int* tile)
 {
-    __shared__ __align__(16) int tile[RANK_SPAN];
-    const int n = meta[META_NTOT];
-    const int b0 = blockIdx.x * 256;
-    if (b0 >= n) return;  // whole block past the end (uniform)
-    const int u = b0 + threadIdx.x;
+    const int u = b0 + (int)threadIdx.x;
     const bool in = u < n;
     const int c0 = tmp_key[b0];
     const int c1 = tmp_key[min(n - 1, b0 + 255)];
@@ -254,8 +319,7 @@ __global__ __launch_bounds__(256) void k_rank(const int* meta, const int* __rest
                 rank += rv > r || (rv == r && base + j < u);
             }
         }
-        if (in) perm[s0 + rank] = tmp_idx[u];
-        return;
+        return s0 + rank;
     }
     // the span of the buckets of the block's first and last thread holds
     // every bucket in between (scatter order is bucket order)
@@ -263,7 +327,7 @@ __global__ __launch_bounds__(256) void k_rank(const int* meta, const int* __rest
     if (c1 != dead_key && span1 - span0 <= RANK_SPAN) {
         for (int j = threadIdx.x; j < span1 - span0; j += 256) tile[j] = tmp_ref[span0 + j];
         __syncthreads();
-        if (!in) return;
+        if (!in) return 0;
         // a live bucket (a cell or a system's removal bucket) holds one
         // system's particles, whose reference indices are distinct: the
         // rank is the count of larger ones, read four at a time
@@ -278,15 +342,11 @@ __global__ __launch_bounds__(256) void k_rank(const int* meta, const int* __rest
             rank += (q.x > r) + (q.y > r) + (q.z > r) + (q.w > r);
         }
         for (; v < ve; ++v) rank += tile[v] > r;
-        perm[s + rank] = tmp_idx[u];
-        return;
+        return s + rank;
     }
-    if (!in) return;
+    if (!in) return 0;
     const int c = tmp_key[u];
-    if (c == dead_key) {
-        perm[u] = tmp_idx[u];
-        return;
-    }
+    if (c == dead_key) return u;
     const int s = cell_start[c], e = cell_start[c + 1];
     const int r = tmp_ref[u];
     int rank = 0;
@@ -295,66 +355,32 @@ __global__ __launch_bounds__(256) void k_rank(const int* meta, const int* __rest
         const int rv = tmp_ref[v];
         rank += rv > r || (rv == r && v < u);
     }
-    perm[s + rank] = tmp_idx[u];
+    return s + rank;
 }
 
-__global__ __launch_bounds__(256) void k_gather(const int* meta, const int* __restrict__ perm,
-                                                const double* __restrict__ src,
-                                                double* __restrict__ dst,
-                                                const int* __restrict__ isrc,
-                                                int* __restrict__ idst, long long cap,
-                                                unsigned skip)
+__global__ __launch_bounds__(256) void k_place(const SysDesc* __restrict__ sysd, int nsys,
+                                               int cells_total, int* sc, int* meta,
+                                               const int* __restrict__ cell_start,
+                                               const int* __restrict__ tmp_idx,
+                                               const int* __restrict__ tmp_key,
+                                               const int* __restrict__ tmp_ref, Move mv)
 {
+    __shared__ __align__(16) int tile[RANK_SPAN];
+    if (blockIdx.x == 0) finalize(sysd, nsys, cells_total, sc, meta, cell_start);
     const int n = meta[META_NTOT];
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    const long long j = perm[k];
-#pragma unroll
-    for (int f = 0; f < NCOL; ++f)
-        if (!((skip >> f) & 1u)) dst[f * cap + k] = src[f * cap + j];
-#pragma unroll
-    for (int f = 0; f < NICOL; ++f) idst[f * cap + k] = isrc[f * cap + j];
-}
-
-// Totals of the build, per system and overall.
-__global__ void k_finalize(const SysDesc* __restrict__ sysd, int nsys, int cells_total, int* sc,
-                           int* meta, const int* cell_start)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s == 0) {
-        const int na = cell_start[cells_total];
-        meta[META_NREM] = meta[META_NTOT] - na;
-        meta[META_N] = na;
-        meta[META_NCELLS] = 0;
-    }
-    if (s >= nsys) return;
-    const SysDesc& d = sysd[s];
-    const int off = cell_start[d.cell_base];
-    const int end = cell_start[d.cell_base + d.g.key_max];
-    sc[SYSCNT * s + SC_OFF] = off;
-    sc[SYSCNT * s + SC_N] = d.live ? end - off : 0;
-    sc[SYSCNT * s + SC_NREM] = cell_start[cells_total + s + 1] - cell_start[cells_total + s];
+    const int b0 = blockIdx.x * 256;
+    if (b0 >= n) return;  // whole block past the end (uniform)
+    const int k = rank_in_bucket(b0, n, cell_start, tmp_key, tmp_ref, cells_total + nsys, tile);
+    const int u = b0 + (int)threadIdx.x;
+    if (u < n) move_particle(mv, tmp_idx[u], tmp_key[u], tmp_ref[u], k, cell_start[cells_total] != n);
 }
 
 // Removal renumbering (src/core.jl:72-81): with the removed reference
 // indices r_1 > r_2 > ... > r_m of a system, particles[r_i] =
-// particles[N+1-i] in turn.  inv maps (system reference base + reference
-// position) to the sorted slot that holds it.
-__global__ __launch_bounds__(256) void k_inv(const int* meta, const int* __restrict__ ref,
-                                             const int* __restrict__ sysid, const int* sc,
-                                             int* inv)
+// particles[N+1-i] in turn.  One thread per system.
+__device__ inline void remove_seq(int s, int cells_total, const int* sc, const int* cell_start,
+                                  int* ref, int* inv)
 {
-    if (meta[META_NREM] == 0) return;
-    const int n = meta[META_NTOT];
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k < n) inv[sc[SYSCNT * sysid[k] + SC_REFBASE] + ref[k]] = k;
-}
-
-__global__ void k_remove_seq(const int* meta, int nsys, int cells_total, const int* sc,
-                             const int* cell_start, int* ref, int* inv)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsys || meta[META_NREM] == 0) return;
     const int m = sc[SYSCNT * s + SC_NREM];
     if (m == 0) return;
     const int first = cell_start[cells_total + s];
@@ -369,7 +395,7 @@ __global__ void k_remove_seq(const int* meta, int nsys, int cells_total, const i
     }
 }
 
-// Rank of local cell lc of a system in brick order: the grid is cut into
+// Local cell at rank lr of a system in brick order: the grid is cut into
 // bricks of BX x BY x BZ cells (BZ = 1 in 2D), the bricks are numbered x
 // fastest, then y, then z, and the cells of a brick x fastest; the bricks
 // on the far faces are cut to the grid, so the ranks are 0 .. key_max - 1.
@@ -379,209 +405,199 @@ __global__ void k_remove_seq(const int* meta, int nsys, int cells_total, const i
 // where a row-major order spreads them over whole rows of the grid.
 constexpr int BRICK_X = 4, BRICK_Y = 4, BRICK_Z = 4, BRICK_2D = 8;
 
-__device__ inline int brick_rank(const Geo& g, int lc)
+__device__ inline int brick_cell(const Geo& g, int lr)
 {
     const int bx = g.L3 > 1 ? BRICK_X : BRICK_2D;
     const int by = g.L3 > 1 ? BRICK_Y : BRICK_2D;
     const int bz = g.L3 > 1 ? BRICK_Z : 1;
-    const int ix = lc % g.L1, r = lc / g.L1;
-    const int iy = r % g.L2, iz = r / g.L2;
-    const int kx = ix / bx, ky = iy / by, kz = iz / bz;
-    const int wx = min(bx, g.L1 - kx * bx);  // extents of this brick
-    const int hy = min(by, g.L2 - ky * by);
+    const int layer = bz * g.L1 * g.L2;  // a layer of bricks (the last may be thinner)
+    const int kz = lr / layer;
     const int hz = min(bz, g.L3 - kz * bz);
-    return kz * bz * g.L1 * g.L2 + ky * by * g.L1 * hz + kx * bx * hy * hz +
-           (ix - kx * bx) + wx * ((iy - ky * by) + hy * (iz - kz * bz));
+    int r = lr - kz * layer;
+    const int row = by * g.L1 * hz;      // a row of bricks
+    const int ky = r / row;
+    const int hy = min(by, g.L2 - ky * by);
+    r -= ky * row;
+    const int brick = bx * hy * hz;
+    const int kx = r / brick;
+    const int wx = min(bx, g.L1 - kx * bx);
+    r -= kx * brick;
+    const int iz = r / (wx * hy), q = r - iz * (wx * hy);
+    const int iy = q / wx, ix = q - iy * wx;
+    return kx * bx + ix + g.L1 * ((ky * by + iy) + g.L2 * (kz * bz + iz));
 }
 
-// 64-candidate chunks one target of global cell c walks: the pair kernels
+// 64-candidate chunks one target of cell c walks: the pair kernels
 // concatenate the cell's stencil ranges and cut the list into chunks of 64.
-// Also places c at its brick rank in order[].
 template <int ROWS>
-__global__ __launch_bounds__(256) void k_cell_chunks(const SysDesc* __restrict__ sysd,
-                                                     const int* __restrict__ cell_sys,
-                                                     int ncells, const int* __restrict__ cell_start,
-                                                     int* chunks, int* order)
+__device__ inline int cell_chunks(const SysDesc& d, const int* cell_start, int lc)
 {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= ncells) return;
-    const SysDesc& d = sysd[cell_sys[c]];
-    const int lc = c - d.cell_base;
-    order[d.cell_base + brick_rank(d.g, lc)] = c;
     int n = 0;
-    if (cell_start[c + 1] > cell_start[c]) {
-        for (int row = 0; row < ROWS; ++row) {
-            Seg seg[2];
-            const int ns = row_segments<ROWS>(d, cell_start, lc, row, seg);
-            for (int q = 0; q < 2; ++q)
-                if (q < ns) n += seg[q].j1 - seg[q].j0;
-        }
+    for (int row = 0; row < ROWS; ++row) {
+        Seg seg[2];
+        const int ns = row_segments<ROWS>(d, cell_start, lc, row, seg);
+        for (int q = 0; q < 2; ++q)
+            if (q < ns) n += seg[q].j1 - seg[q].j0;
     }
-    chunks[c] = (n + 63) / 64;
+    return (n + 63) / 64;
 }
 
 // Tile table, in brick order: tile k of the cell c at rank r covers targets
-// cell_start[c] + k*T ...; its pair masks start at mask_start[r] +
-// k * chunks[c] * T, its kept-candidate list at 64 / T times that.
-__global__ __launch_bounds__(256) void k_tiles(const int* __restrict__ cell_start,
-                                               const int* __restrict__ tile_start,
-                                               const int* __restrict__ chunks,
-                                               const int* __restrict__ order,
-                                               const unsigned long long* __restrict__ mask_start,
-                                               int ncells, int T, long long mask_cap,
-                                               long long kept_cap, int4* tiles, int* meta,
-                                               unsigned long long* mask_total)
+// cell_start[c] + k*T ...; its pair masks start at the mask words of the
+// tiles before it (chunks * T words each), its kept-candidate list at 64 / T
+// times that.  Each thread takes TT_CELLS consecutive ranks; tiles and mask
+// words are scanned together, by two waves of each block (chained blocks).
+// The first block also clears the tile queues and replays the removals.
+static constexpr int TT_CELLS = 4;
+static constexpr int TT_TILE = 256 * TT_CELLS;
+
+template <int ROWS>
+__global__ __launch_bounds__(256) void k_tile_table(
+    const SysDesc* __restrict__ sysd, const int* __restrict__ cell_sys, int ncells,
+    const int* __restrict__ cell_start, int T, long long mask_cap, long long kept_cap, int4* tiles,
+    int* meta, unsigned long long* mask_total, unsigned long long* stat_tiles,
+    unsigned long long* stat_words, unsigned long long* ticket, int* queue, int nsys, int removal,
+    const int* sc, int* ref, int* inv)
 {
+    __shared__ unsigned long long prefix[2];
     __shared__ int with_tiles;
     if (threadIdx.x == 0) with_tiles = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        meta[META_NTILES] = tile_start[ncells];
-        const unsigned long long need = mask_start[ncells];
-        *mask_total = need;
-        meta[META_MASK_OK] = (long long)need <= mask_cap ? 1 : 0;
-        // 64 kept-candidate entries per chunk of a tile, T mask words
-        meta[META_KEPT_OK] = (long long)(need / T * 64) <= kept_cap ? 1 : 0;
+    const int b = chain_ticket(ticket);  // (a block barrier)
+    if (b == 0) {
+        if (threadIdx.x < NQUEUE * NQUEUE_SETS) queue[threadIdx.x * QSTRIDE] = 0;
+        if (removal && meta[META_NREM] != 0)
+            for (int s = threadIdx.x; s < nsys; s += 256)
+                remove_seq(s, ncells, sc, cell_start, ref, inv);
     }
-    __syncthreads();
-    // cells with tiles: counted per block, one global atomic per block (a
-    // single address serialises its atomics)
-    int n = 0;
-    for (int r = blockIdx.x * 256 + threadIdx.x; r < ncells; r += gridDim.x * 256) {
-        const int t0 = tile_start[r], nt = tile_start[r + 1] - t0;
-        n += nt > 0;
-        const int c = order[r];
-        const int cs = cell_start[c];
-        const long long words = (long long)chunks[c] * T;
-        for (int t = 0; t < nt; ++t) {
-            const unsigned long long base = mask_start[r] + (unsigned long long)(t * words);
-            tiles[t0 + t] = make_int4(c, cs + t * T, (int)(unsigned)(base & 0xffffffffull),
-                                      (int)(base >> 32));
-        }
-    }
-    if (n) atomicAdd(&with_tiles, n);
-    __syncthreads();
-    if (threadIdx.x == 0 && with_tiles) atomicAdd(&meta[META_NCELLS], with_tiles);
-}
-
-// Bounding box of each tile's targets (absolute FP64), read by the pair
-// kernels to cull candidates.  A wave covers 64 / T tiles at a time, one
-// lane per target.  The coordinates go through LDS; of the T lanes of a
-// tile, G = T / 8 lanes per bound (c < 6: min x, max x, min y, ...) reduce
-// eight coordinates each and combine in log2(G) shuffle steps.  Targets
-// past the cell's end take the first target's place; NaN coordinates are
-// ignored (fmin/fmax).
-template <bool FLAT>
-__global__ __launch_bounds__(256) void k_tile_boxes(const int4* __restrict__ tiles,
-                                                    const int* __restrict__ cell_start,
-                                                    const int* meta, const double* __restrict__ x,
-                                                    const double* __restrict__ y,
-                                                    const double* __restrict__ z, int T,
-                                                    double* boxes)
-{
-    __shared__ double xs[4][3][64];
-    const int ntiles = meta[META_NTILES];
-    const int lane = threadIdx.x & 63;
-    double(*w)[64] = xs[threadIdx.x >> 6];
-    const int per_wave = 64 / T, G = T / 8;
-    const int tw = lane / T, lt = lane % T;  // tile in the wave, target in the tile
-    const int c = lt / G, j = lt % G, axis = c >> 1;
-    const bool lo = (c & 1) == 0;
-    const long long per_block = 4ll * per_wave, step = (long long)gridDim.x * per_block;
-    // the block's four waves step together (block barriers)
-    for (long long b = (long long)blockIdx.x * per_block; b < ntiles; b += step) {
-        const long long i = b + (threadIdx.x >> 6) * per_wave + tw;
-        if (i < ntiles) {
-            const int4 td = tiles[i];
-            const int p = td.y + lt;
-            const int pp = p < cell_start[td.x + 1] ? p : td.y;
-            w[0][lane] = x[pp];
-            w[1][lane] = y[pp];
-            w[2][lane] = FLAT ? 0.0 : z[pp];
-        }
-        __syncthreads();
-        double v = 0.0;
-        if (c < 6) {
-            const int k0 = tw * T + 8 * j;
-            v = w[axis][k0];
-            for (int k = 1; k < 8; ++k) {
-                const double u = w[axis][k0 + k];
-                v = lo ? fmin(v, u) : fmax(v, u);
+    int cell[TT_CELLS], nt[TT_CELLS];
+    long long words[TT_CELLS];  // of one tile
+    unsigned tsum = 0;
+    unsigned long long wsum = 0;
+    int ncell = 0;
+#pragma unroll
+    for (int k = 0; k < TT_CELLS; ++k) {
+        const int r = b * TT_TILE + (int)threadIdx.x * TT_CELLS + k;
+        cell[k] = nt[k] = 0;
+        words[k] = 0;
+        if (r < ncells) {
+            const SysDesc& d = sysd[cell_sys[r]];
+            const int lc = brick_cell(d.g, r - d.cell_base);
+            const int c = d.cell_base + lc;
+            const int n = cell_start[c + 1] - cell_start[c];
+            cell[k] = c;
+            if (n > 0) {
+                nt[k] = (n + T - 1) / T;
+                words[k] = (long long)cell_chunks<ROWS>(d, cell_start, lc) * T;
+                ++ncell;
             }
         }
-        for (int o = 1; o < G; o <<= 1) {
-            const double u = __shfl_xor(v, o);
-            v = lo ? fmin(v, u) : fmax(v, u);
-        }
-        if (i < ntiles && c < 6 && j == 0) boxes[6 * i + c] = v;
-        __syncthreads();
+        tsum += (unsigned)nt[k];
+        wsum += (unsigned long long)(nt[k] * words[k]);
     }
+    if (ncell) atomicAdd(&with_tiles, ncell);
+    unsigned ttot;
+    unsigned long long wtot;
+    unsigned trun = block_incl_scan(tsum, ttot) - tsum;
+    unsigned long long wrun = block_incl_scan(wsum, wtot) - wsum;
+    if (threadIdx.x < 128) {  // the first wave chains the tiles, the second the words
+        const int w = threadIdx.x >> 6;
+        const unsigned long long p = chain_prefix(w ? stat_words : stat_tiles, b,
+                                                  w ? wtot : (unsigned long long)ttot);
+        if ((threadIdx.x & 63) == 0) prefix[w] = p;
+    }
+    __syncthreads();
+    trun += (unsigned)prefix[0];
+    wrun += prefix[1];
+    if (threadIdx.x == 0) {
+        if (with_tiles) atomicAdd(&meta[META_NCELLS], with_tiles);
+        if (b == (int)gridDim.x - 1) {
+            const unsigned long long need = prefix[1] + wtot;
+            meta[META_NTILES] = (int)((unsigned)prefix[0] + ttot);
+            *mask_total = need;
+            meta[META_MASK_OK] = (long long)need <= mask_cap ? 1 : 0;
+            // 64 kept-candidate entries per chunk of a tile, T mask words
+            meta[META_KEPT_OK] = (long long)(need / T * 64) <= kept_cap ? 1 : 0;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < TT_CELLS; ++k) {
+        const int cs = nt[k] > 0 ? cell_start[cell[k]] : 0;
+        for (int t = 0; t < nt[k]; ++t) {
+            tiles[trun++] = make_int4(cell[k], cs + t * T, (int)(unsigned)(wrun & 0xffffffffull),
+                                      (int)(wrun >> 32));
+            wrun += (unsigned long long)words[k];
+        }
+    }
+}
+
+// State words of the scans and the count of cells with tiles, cleared for a
+// tile table built apart from a cell list.
+__global__ __launch_bounds__(256) void k_reset_scans(unsigned long long* stat, int nstat, int* meta)
+{
+    for (int j = blockIdx.x * 256 + threadIdx.x; j < nstat; j += gridDim.x * 256) stat[j] = 0ull;
+    if (blockIdx.x == 0 && threadIdx.x == 0) meta[META_NCELLS] = 0;
 }
 
 // ------------------------------------------------------------ host side --
 static inline unsigned nblocks(long long n, int b) { return (unsigned)((n + b - 1) / b); }
 
-void enqueue_tiles(sph_system* s)
+// State words of the build's scans, for `cells` buckets: the counts, tiles
+// and mask words of each block, then one ticket per scan.
+static inline int stat_blocks(long long cells) { return (int)(cells / TT_TILE) + 2; }
+long long scan_state_needed(long long cells) { return 3ll * stat_blocks(cells) + 2; }
+
+static void enqueue_tile_table(sph_system* s, int removal)
 {
     const int ncells = (int)s->cells_total;
-    const unsigned nbc = nblocks(ncells + 1, 256);
-    if (s->rows == 3)
-        k_cell_chunks<3><<<nbc, 256, 0, s->stream>>>(s->sysd, s->cell_sys, ncells, s->cell_start,
-                                                     s->cell_chunks, s->cell_order);
-    else
-        k_cell_chunks<9><<<nbc, 256, 0, s->stream>>>(s->sysd, s->cell_sys, ncells, s->cell_start,
-                                                     s->cell_chunks, s->cell_order);
-    scan(s, SrcTiles{s->cell_start, s->cell_order, ncells, s->tile_T}, ncells + 1, s->tile_start,
-         s->scan_part);
-    scan(s, SrcMaskWords{s->tile_start, s->cell_chunks, s->cell_order, ncells, s->tile_T},
-         ncells + 1, s->mask_start, s->scan_part64);
-    k_tiles<<<nbc < 256 ? nbc : 256, 256, 0, s->stream>>>(s->cell_start, s->tile_start,
-                                        s->cell_chunks, s->cell_order,
-                                        s->mask_start, ncells, s->tile_T,
-                                        s->masks ? s->mask_cap : 0,
-                                        s->kept && (s->kept_rg || !s->periodic) ? s->kept_cap : 0,
-                                        s->tiles, s->meta,
-                                        s->mask_total);
-    const double* c = s->cols[s->cur];
-    const long long cap = s->cap;
-    const unsigned nbt = 2048;  // waves loop over the tiles
-    auto boxes = s->flat ? k_tile_boxes<true> : k_tile_boxes<false>;
-    boxes<<<nbt, 256, 0, s->stream>>>(s->tiles, s->cell_start, s->meta, c + C_X * cap,
-                                      c + C_Y * cap, c + C_Z * cap, s->tile_T, s->boxes);
+    const unsigned nb = nblocks(ncells, TT_TILE);
+    const int sb = stat_blocks(s->cells_cap);
+    unsigned long long* stat = s->scan_state;
+    auto k = s->rows == 3 ? k_tile_table<3> : k_tile_table<9>;
+    k<<<nb, 256, 0, s->stream>>>(s->sysd, s->cell_sys, ncells, s->cell_start, s->tile_T,
+                                 s->masks ? s->mask_cap : 0,
+                                 s->kept && (s->kept_rg || !s->periodic) ? s->kept_cap : 0,
+                                 s->tiles, s->meta, s->mask_total, stat + sb, stat + 2 * sb,
+                                 stat + 3 * sb + 1, s->queue, (int)s->sys_host.size(), removal,
+                                 s->sys_cnt, s->icols[s->cur] + I_REF * s->cap, s->inv);
+}
+
+// The tile table of the current cell list for another tile size.
+void enqueue_tiles(sph_system* s)
+{
+    const int nstat = (int)scan_state_needed(s->cells_cap);
+    k_reset_scans<<<nblocks(nstat, 256), 256, 0, s->stream>>>(s->scan_state, nstat, s->meta);
+    enqueue_tile_table(s, 0);
 }
 
 // skip_cols: columns (bit C_*) the caller rewrites for every particle before
-// reading them; the gather leaves their values in the new order undefined.
-void enqueue_build(sph_system* s, unsigned skip_cols)
+// reading them (skip_a: the acceleration of every fluid particle); they are
+// not moved, and their values in the new order are undefined.
+void enqueue_build(sph_system* s, unsigned skip_cols, int skip_a)
 {
     hipStream_t st = s->stream;
     const long long cap = s->cap;
     const int nsys = (int)s->sys_host.size();
     const int ncells = (int)s->cells_total;
-    const long long nbuckets = s->cells_total + nsys + 1;
+    const int nbuckets = (int)(s->cells_total + nsys + 1);
     const unsigned nb = nblocks(s->n > 0 ? s->n : 1, 256);
+    const int sb = stat_blocks(s->cells_cap);
     double* c = s->cols[s->cur];
     int* ic = s->icols[s->cur];
-    k_sys_prep<<<1, 256, 0, st>>>(nsys, s->sys_cnt, s->meta);
-    k_fill_u32<<<nblocks(nbuckets, 256), 256, 0, st>>>(s->cnt, 0u, nbuckets);
+    unsigned long long* stat = s->scan_state;
     k_keys<<<nb, 256, 0, st>>>(s->sysd, nsys, ncells, c + C_X * cap, c + C_Y * cap,
                                c + C_Z * cap, ic + I_SYS * cap, s->meta, ic + I_KEY * cap,
-                               s->slot, s->cnt);
-    scan(s, SrcCount{s->cnt}, (int)nbuckets, s->cell_start, s->scan_part);
+                               s->slot, s->cnt, s->sys_cnt, stat,
+                               (int)scan_state_needed(s->cells_cap));
+    k_scan_counts<<<nblocks(nbuckets + 1, CSCAN_TILE), 256, 0, st>>>(s->cnt, nbuckets, s->cell_start,
+                                                                     stat, stat + 3 * sb);
     k_scatter<<<nb, 256, 0, st>>>(s->meta, ic + I_KEY * cap, s->slot, ic + I_REF * cap,
                                   s->cell_start, s->tmp_idx, s->tmp_key, s->tmp_ref);
-    k_rank<<<nb, 256, 0, st>>>(s->meta, s->cell_start, s->tmp_idx, s->tmp_key, s->tmp_ref,
-                               s->perm, ncells + nsys);
-    k_gather<<<nb, 256, 0, st>>>(s->meta, s->perm, c, s->cols[s->cur ^ 1], ic,
-                                 s->icols[s->cur ^ 1], cap, skip_cols);
+    const Move mv{c, s->cols[s->cur ^ 1], ic, s->icols[s->cur ^ 1], cap, skip_cols, skip_a,
+                  s->sys_cnt, s->inv};
+    k_place<<<nb, 256, 0, st>>>(s->sysd, nsys, ncells, s->sys_cnt, s->meta, s->cell_start,
+                                s->tmp_idx, s->tmp_key, s->tmp_ref, mv);
     s->cur ^= 1;
-    int* ref = s->icols[s->cur] + I_REF * cap;
-    int* sysid = s->icols[s->cur] + I_SYS * cap;
-    k_finalize<<<nblocks(nsys, 64), 64, 0, st>>>(s->sysd, nsys, ncells, s->sys_cnt, s->meta,
-                                                  s->cell_start);
-    k_inv<<<nb, 256, 0, st>>>(s->meta, ref, sysid, s->sys_cnt, s->inv);
-    k_remove_seq<<<nblocks(nsys, 64), 64, 0, st>>>(s->meta, nsys, ncells, s->sys_cnt,
-                                                    s->cell_start, ref, s->inv);
-    enqueue_tiles(s);
+    enqueue_tile_table(s, 1);
 }
 
 }  // namespace sph

@@ -565,10 +565,7 @@ __device__ inline void tile32(const PairCtx& c, int tile, int out_col, bool load
     if (!use_kept) {
         // RN(x - ox) is monotonic in x: the box of the relative positions
         // is the relative box
-        const Box<double> b = ld_const(reinterpret_cast<const Box<double>*>(c.boxes) + tile);
-        box.x0 = (float)(b.x0 - ox); box.x1 = (float)(b.x1 - ox);
-        box.y0 = (float)(b.y0 - oy); box.y1 = (float)(b.y1 - oy);
-        box.z0 = (float)(b.z0 - oz); box.z1 = (float)(b.z1 - oz);
+        box = tile_box<FLAT>(tg.x, tg.y, tg.z);
         nr = build_cands<ROWS, PERIODIC>(d, c.cell_start, lc, L, total);
     }
     // matrix-core test: centre of the box and the targets' operands

@@ -487,7 +487,7 @@ __device__ inline void tile64(const PairCtx& c, int tile, bool load_masks, bool 
     const int nk = use_kept ? ld_const(c.kept_n + tile) : 0;
     int total = 0, nr = 0;
     Box<double> box{};
-    if (!use_kept) box = ld_const(reinterpret_cast<const Box<double>*>(c.boxes) + tile);
+    if (!use_kept) box = tile_box<FLAT>(tg.x, tg.y, tg.z);
     // (periodic systems need the ranges' image shifts in either case)
     if (!use_kept || PERIODIC) nr = build_cands<ROWS, PERIODIC>(d, c.cell_start, lc, L, total);
     // matrix-core test: centre of the box and the targets' operands

@@ -382,6 +382,71 @@ __device__ inline void test_chunk(const TestTile<T>& tt, float x, float y, float
     m &= ~unsure;
 }
 
+// --------------------------------------------------------- wave reductions --
+// Inclusive prefix sum of v over the wave's lanes, in six DPP steps: the
+// row shifts by 1, 2, 4 and 8 lanes scan each row of 16 lanes, then the
+// broadcast of lane 15 carries row 0's total into row 1 and row 2's into
+// row 3, and the broadcast of lane 31 carries rows 0-1's total into rows 2
+// and 3.  Lanes a step does not write add the 0 given as the old value.
+// Every lane of the wave must be active.
+__device__ inline int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return v;
+}
+
+// Copy of v from the lane a DPP step reads; lanes the step does not write
+// keep their own.
+template <int CTRL, int ROW_MASK>
+__device__ inline float dpp_own(float v)
+{
+    const int b = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(b, b, CTRL, ROW_MASK, 0xf, false));
+}
+
+template <int CTRL, int ROW_MASK>
+__device__ inline double dpp_own(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)b, hi = (int)(b >> 32);
+    const int l = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xf, false);
+    const int h = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xf, false);
+    return __longlong_as_double((long long)(((unsigned long long)(unsigned)h << 32) | (unsigned)l));
+}
+
+__device__ inline float lane63(float v)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+__device__ inline double lane63(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, 63);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Smallest and largest v over the wave (uniform); the steps of wave_scan.
+template <class V>
+__device__ inline void wave_bounds(V v, V& lo, V& hi)
+{
+    V a = v, b = v;
+    a = fmin(a, dpp_own<0x111, 0xf>(a)); b = fmax(b, dpp_own<0x111, 0xf>(b));
+    a = fmin(a, dpp_own<0x112, 0xf>(a)); b = fmax(b, dpp_own<0x112, 0xf>(b));
+    a = fmin(a, dpp_own<0x114, 0xf>(a)); b = fmax(b, dpp_own<0x114, 0xf>(b));
+    a = fmin(a, dpp_own<0x118, 0xf>(a)); b = fmax(b, dpp_own<0x118, 0xf>(b));
+    a = fmin(a, dpp_own<0x142, 0xa>(a)); b = fmax(b, dpp_own<0x142, 0xa>(b));
+    a = fmin(a, dpp_own<0x143, 0xc>(a)); b = fmax(b, dpp_own<0x143, 0xc>(b));
+    lo = lane63(a);
+    hi = lane63(b);
+}
+
 // ------------------------------------------------------------ candidates --
 // The candidate ranges of a tile: its cell's stencil rows, concatenated.
 // pref[i] candidates precede range i; a chunk's slot l holds candidate
@@ -402,36 +467,45 @@ struct Cands {
     int self0[MAXR];
 };
 
-// Uniform work (every lane computes the same values); lane 0 writes.
-// Returns the number of ranges; *total receives the candidate count.
+// Ranges of the tile's candidate list, one lane per range (empty ones are
+// kept in place): the lanes' loads of the row ends overlap, and a prefix sum
+// concatenates the rows.  Returns the number of ranges; *total receives the
+// candidate count.  (One row after the other, each waiting for its loads,
+// took ~55 instructions per row and 2-4 us per tile.)
 template <int ROWS, bool PERIODIC, int NQ>
 __device__ inline int build_cands(const SysDesc& d, const int* cell_start, int lc,
                                   Cands<ROWS, PERIODIC, NQ>& L, int& total)
 {
-    const bool w = __lane_id() == 0;
-    int n = 0, tot = 0;
-    for (int row = 0; row < ROWS; ++row) {
+    constexpr int NR = PERIODIC ? 2 * ROWS : ROWS;
+    const int lane = __lane_id();
+    int len = 0;
+    Seg g{};
+    if (lane < NR) {
         Seg segs[2];
-        const int ns = row_segments<ROWS, PERIODIC>(d, cell_start, lc, row, segs);
-        for (int k = 0; k < 2; ++k) {
-            if (k < ns) {
-                if (w) {
-                    L.j0[n] = segs[k].j0;
-                    L.pref[n] = tot;
-                    if constexpr (PERIODIC) {
-                        L.sx[n] = segs[k].sx;
-                        L.sy[n] = segs[k].sy;
-                        L.sz[n] = segs[k].sz;
-                    }
-                }
-                tot += segs[k].j1 - segs[k].j0;
-                ++n;
-            }
+        const int k = PERIODIC ? lane & 1 : 0;
+        const int ns = row_segments<ROWS, PERIODIC>(d, cell_start, lc, PERIODIC ? lane >> 1 : lane,
+                                                    segs);
+        // field by field: a selected struct would live in scratch
+        g.j0 = k ? segs[1].j0 : segs[0].j0;
+        g.j1 = k ? segs[1].j1 : segs[0].j1;
+        g.sx = k ? segs[1].sx : segs[0].sx;
+        g.sy = segs[0].sy;
+        g.sz = segs[0].sz;
+        if (k < ns) len = g.j1 - g.j0;
+    }
+    const int incl = wave_scan(len);
+    total = __builtin_amdgcn_readlane(incl, 63);
+    if (lane < NR) {
+        L.j0[lane] = g.j0;
+        L.pref[lane] = incl - len;
+        if constexpr (PERIODIC) {
+            L.sx[lane] = g.sx;
+            L.sy[lane] = g.sy;
+            L.sz[lane] = g.sz;
         }
     }
-    if (w) L.pref[n] = tot;
-    total = tot;
-    return n;
+    if (lane == 0) L.pref[NR] = total;
+    return NR;
 }
 
 // Slot of chunk `base` that holds candidate g (g < total): its range and
@@ -507,13 +581,26 @@ __device__ inline void drop_self(const Cands<ROWS, PER, NQ>& L, int nself, int h
     }
 }
 
-// Bounding box of a tile's targets, computed with the tile table in absolute
-// FP64 coordinates; the mixed kernels convert it to FP32 relative to the
-// tile's first target.
+// Bounding box of a tile's targets: absolute in the FP64 kernels, relative to
+// the tile's first target in the mixed ones.
 template <class V>
 struct Box {
     V x0, x1, y0, y1, z0, z1;
 };
+
+// The box of the lanes' targets (lanes without one hold the first): a few
+// DPP steps per tile, where a kernel of its own that read the positions again
+// and stored 48 bytes per tile took 50 us per 5.75M-particle build.
+template <bool FLAT, class V>
+__device__ inline Box<V> tile_box(V x, V y, V z)
+{
+    Box<V> b;
+    wave_bounds(x, b.x0, b.x1);
+    wave_bounds(y, b.y0, b.y1);
+    b.z0 = b.z1 = V(0);
+    if (!FLAT) wave_bounds(z, b.z0, b.z1);
+    return b;
+}
 
 // Squared distance of (x, y, z) to the box (0 inside), evaluated in the
 // predicate's operation order.
@@ -622,23 +709,6 @@ __device__ inline V shfl_value(const V& v, int src)
 #pragma unroll
     for (unsigned i = 0; i < sizeof(V) / 4; ++i) b[i] = __shfl(a[i], src);
     return r;
-}
-
-// Inclusive prefix sum of v over the wave's lanes, in six DPP steps: the
-// row shifts by 1, 2, 4 and 8 lanes scan each row of 16 lanes, then the
-// broadcast of lane 15 carries row 0's total into row 1 and row 2's into
-// row 3, and the broadcast of lane 31 carries rows 0-1's total into rows 2
-// and 3.  Lanes a step does not write add the 0 given as the old value.
-// Every lane of the wave must be active.
-__device__ inline int wave_scan(int v)
-{
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
-    return v;
 }
 
 // Sum of v over the wave (uniform).

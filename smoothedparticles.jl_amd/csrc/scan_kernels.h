@@ -1,5 +1,6 @@
-// Exclusive device-wide scan shared by the cell-list build (cells.hip) and
-// the device lattice generator (generate.hip).
+// Device-wide exclusive scans: the chained scan of the cell-list build
+// (cells.hip) and the three-launch scan of the device lattice generator
+// (generate.hip).
 #pragma once
 
 #include "sph_internal.h"
@@ -9,7 +10,7 @@ namespace sph {
 static constexpr int SCAN_ITEMS = 16;
 static constexpr int SCAN_TILE = 256 * SCAN_ITEMS;
 
-// Exclusive device-wide scan, three launches: per-block sums, one block
+// Three launches: per-block sums, one block
 // scanning the block sums, per-block scans plus offset.  V is unsigned or
 // unsigned long long.
 template <class V>
@@ -38,6 +39,58 @@ __device__ inline V block_incl_scan(V v, V& total)
     total = wsum[0] + wsum[1] + wsum[2] + wsum[3];
     __syncthreads();
     return w + off;
+}
+
+// Chained scan, one launch: every block scans its own part and takes the sum
+// of the parts before it from their state words.  A state word holds a value
+// and, in its top two bits, whether it is the block's own sum or the sum up
+// to and including the block; it is written and read as one 64-bit atomic,
+// so it needs no fence (values stay below 2^62).  The words and the ticket
+// are cleared before the launch.
+static constexpr unsigned long long CHAIN_SUM = 1ull << 62, CHAIN_PREFIX = 2ull << 62;
+static constexpr unsigned long long CHAIN_VALUE = CHAIN_SUM - 1;
+
+// The block's place in the chain.  Places are handed out in the order in
+// which the blocks start, so every block before one that waits is running or
+// done, and the wait ends.  Contains a block barrier.
+__device__ inline int chain_ticket(unsigned long long* ticket)
+{
+    __shared__ int place;
+    if (threadIdx.x == 0) place = (int)atomicAdd(ticket, 1ull);
+    __syncthreads();
+    return place;
+}
+
+// Sum of the blocks before place b, whose own sum is `sum`; called by one
+// whole wave, the same value in every lane.
+__device__ inline unsigned long long chain_prefix(unsigned long long* stat, int b,
+                                                  unsigned long long sum)
+{
+    const int lane = __lane_id();
+    if (lane == 0)
+        __hip_atomic_store(&stat[b], (b == 0 ? CHAIN_PREFIX : CHAIN_SUM) | sum, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long before = 0;
+    for (int p = b - 1; p >= 0; p -= 64) {
+        // lane l looks at block p - l (blocks before the first: an empty prefix)
+        unsigned long long v;
+        do {
+            v = p - lane >= 0 ? __hip_atomic_load(&stat[p - lane], __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : CHAIN_PREFIX;
+        } while (!__all((v & ~CHAIN_VALUE) != 0ull));
+        const unsigned long long whole = __ballot((v & CHAIN_PREFIX) != 0ull);
+        const int last = whole ? __ffsll((long long)whole) - 1 : 63;
+        unsigned long long t = lane <= last ? v & CHAIN_VALUE : 0ull;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o);
+        before += t;
+        if (whole) break;
+    }
+    if (lane == 0 && b > 0)
+        __hip_atomic_store(&stat[b], CHAIN_PREFIX | (before + sum), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    return before;
 }
 
 template <class Src>

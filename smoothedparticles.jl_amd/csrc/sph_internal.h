@@ -106,7 +106,6 @@ struct PairCtx {
     int* kept;                // kept candidates of each tile (64 per mask chunk)
     unsigned char* kept_rg;   // their candidate ranges (periodic systems: image shift)
     int* kept_n;              // kept candidates per tile
-    const double* boxes;      // bounding box of each tile's targets (6 doubles)
     int mask_mode;
     int masks_mixed;          // the masks were stored by a mixed-precision pass
     const int* cell_start;
@@ -133,6 +132,9 @@ struct PairCtx {
 // helps the other queues.
 static constexpr int NQUEUE = 8;
 static constexpr int QSTRIDE = 32;
+// Sets of queue heads: a cell build clears them all, and the first passes
+// after it take one each (the others clear set 0 first).
+static constexpr int NQUEUE_SETS = 2;
 
 // The pair passes count accepted pairs and distance tests in CNT_COPIES
 // copies of the counters, each on its own 128-byte line: a wave adds to copy
@@ -313,34 +315,27 @@ struct sph_system {
 
     int* meta;           // device counters
     int* meta_host;      // pinned mirror
-    int* queue;          // NQUEUE * QSTRIDE ints: tile-queue heads
+    int* queue;          // NQUEUE_SETS * NQUEUE * QSTRIDE ints: tile-queue heads
     unsigned long long* pair_counter;       // CNT_SLOTS: density pairs, force pairs, tests
     unsigned long long* pair_counter_host;  // pinned mirror
 
     // build scratch
-    unsigned* cnt;       // buckets
+    unsigned* cnt;       // buckets (all zero between builds)
     int* cell_start;     // buckets + 1
-    int* tile_start;     // cells + 1, by brick rank (cell_order)
-    unsigned* scan_part; // scan partials
-    long long scan_part_n;
+    unsigned long long* scan_state;  // state words of the build's scans
+    long long scan_state_n;
     int* slot;           // cap
     int* tmp_idx;        // cap
     int* tmp_key;        // cap
     int* tmp_ref;        // cap
-    int* perm;           // cap
     int* inv;            // cap
     int4* tiles;         // tile bound
     long long tile_cap;
-    int* cell_chunks;    // cells: 64-candidate chunks of a target of the cell
-    int* cell_order;     // cells: global cell at each brick rank (tile-table order)
-    unsigned long long* mask_start;  // cells + 1, by brick rank: first mask word
-    unsigned long long* scan_part64;
     unsigned long long* masks;       // pair masks of the current cell list
     int* kept;                       // kept-candidate lists of the tiles (64 per chunk)
     long long kept_cap;              // entries allocated
     unsigned char* kept_rg;          // kept_cap entries when a system is periodic, else null
     int* kept_n;                     // tile_cap: kept candidates per tile
-    double* boxes;                   // 6 * tile_cap: bounding boxes of the tiles' targets
     long long mask_cap;              // words allocated
     unsigned long long* mask_total;  // device: words needed (1 value)
     bool masks_valid;                // masks match the cell list and positions
