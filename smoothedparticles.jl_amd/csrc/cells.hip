@@ -559,6 +559,7 @@ static void enqueue_tile_table(sph_system* s, int removal)
                                  s->tiles, s->meta, s->mask_total, stat + sb, stat + 2 * sb,
                                  stat + 3 * sb + 1, s->queue, (int)s->sys_host.size(), removal,
                                  s->sys_cnt, s->icols[s->cur] + I_REF * s->cap, s->inv);
+    s->queue_used = 0;
 }
 
 // The tile table of the current cell list for another tile size.

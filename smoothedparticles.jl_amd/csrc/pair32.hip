@@ -795,15 +795,15 @@ static void launch_tile_k(int op, const PairCtx& c, int grid, hipStream_t st)
 }
 
 // A pass that loads the masks launches the kernel for the kept-list path and
-// the general one; the device's mask state picks which of them works.  The
+// the general one, or the one the host knows to work (Loading).  The
 // density, count, emit and digest passes never load kept lists.
 template <int ROWS, bool FLAT, bool PER, int T>
 static void launch_tile(int op, const PairCtx& c, int grid, hipStream_t st)
 {
     const bool loads = c.mask_mode == MASK_LOAD && op != P_DENSITY && op != P_DENSITY_RHO0 &&
                        op != P_COUNT && op != P_EMIT && op != P_DIGEST;
-    if (loads) launch_tile_k<ROWS, FLAT, PER, T, true>(op, c, grid, st);
-    launch_tile_k<ROWS, FLAT, PER, T, false>(op, c, grid, st);
+    if (loads && c.loading != LOAD_GENERAL) launch_tile_k<ROWS, FLAT, PER, T, true>(op, c, grid, st);
+    if (!loads || c.loading != LOAD_KEPT) launch_tile_k<ROWS, FLAT, PER, T, false>(op, c, grid, st);
 }
 
 template <int ROWS, bool FLAT, bool PER>

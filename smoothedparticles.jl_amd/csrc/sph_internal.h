@@ -123,7 +123,13 @@ struct PairCtx {
     int self;                 // add the self term (density)
     int overwrite;            // write instead of accumulate
     int only_flagged;         // skip systems whose pass_on is 0
+    int loading;              // kernels of a loading pass: LOAD_* (the device decides, or known)
 };
+
+// A pass that loads the masks launches the kernel for masks with kept lists
+// and the general one, and the device's mask state picks the one that works,
+// unless the host knows that state.
+enum Loading { LOAD_ASK = 0, LOAD_KEPT = 1, LOAD_GENERAL = 2 };
 
 // Tile queues of the pair kernels: the tiles are split into NQUEUE
 // contiguous ranges with one head counter each (on its own 128-byte line);
@@ -281,6 +287,17 @@ void launch_candidates(int rows, const PairCtx& c, const int* key, unsigned long
 
 }  // namespace sph
 
+namespace sph {
+// What the host reads back at its synchronisation points, written by
+// k_report (and the reductions) straight into pinned host memory.
+struct Report {
+    int meta[META_SLOTS];
+    unsigned long long mask_total;
+    unsigned long long pairs[3];  // pair counters, summed over their copies
+    double red[3];
+};
+}  // namespace sph
+
 // The opaque handle of sph.h / sph_batch.h: a batch of systems.
 struct sph_system {
     int precision;
@@ -314,10 +331,10 @@ struct sph_system {
     int cur;
 
     int* meta;           // device counters
-    int* meta_host;      // pinned mirror
+    sph::Report* report; // pinned
     int* queue;          // NQUEUE_SETS * NQUEUE * QSTRIDE ints: tile-queue heads
-    unsigned long long* pair_counter;       // CNT_SLOTS: density pairs, force pairs, tests
-    unsigned long long* pair_counter_host;  // pinned mirror
+    unsigned queue_used; // bit per set: used since a build cleared them
+    unsigned long long* pair_counter;  // CNT_SLOTS: density pairs, force pairs, tests
 
     // build scratch
     unsigned* cnt;       // buckets (all zero between builds)
@@ -346,7 +363,6 @@ struct sph_system {
     double* stage;       // 9 * cap (field IO)
     double* red_part;    // reduction partials
     long long red_part_n;
-    double* red_out;     // 3 reduction results
     unsigned long long step_pairs[3];  // density pairs, force pairs, density tests  // pair counts of the last sph_step
 
     // batch bookkeeping (host only)

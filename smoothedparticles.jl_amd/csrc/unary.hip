@@ -558,6 +558,33 @@ __global__ __launch_bounds__(256) void k_append(int n0, int m, int ref0, int sys
     icols[I_SYS * cap + k] = sys;
 }
 
+// The host's view of the device counters, into pinned memory (one block).
+__global__ __launch_bounds__(256) void k_report(const int* __restrict__ meta,
+                                                const unsigned long long* __restrict__ mask_total,
+                                                const unsigned long long* __restrict__ counters,
+                                                const int* __restrict__ sys_cnt, int nsys,
+                                                Report* rep, int* sys_cnt_host)
+{
+    const int t = (int)threadIdx.x;
+    if (t < META_SLOTS) rep->meta[t] = meta[t];
+    if (t == META_SLOTS) rep->mask_total = *mask_total;
+    for (int i = t; i < SYSCNT * nsys; i += 256) sys_cnt_host[i] = sys_cnt[i];
+    if (t >= 64 && t < 128) {  // the second wave sums the copies of the counters
+        for (int k = 0; k < 3; ++k) {
+            unsigned long long v = counters[(t - 64) * CNT_STRIDE + k];
+            for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+            if (t == 64) rep->pairs[k] = v;
+        }
+    }
+}
+
+__global__ void k_set_sys(SysDesc* sysd, SysDesc d)
+{
+    const int* src = reinterpret_cast<const int*>(&d);
+    int* dst = reinterpret_cast<int*>(sysd);
+    for (unsigned i = threadIdx.x; i < sizeof(SysDesc) / 4; i += 64) dst[i] = src[i];
+}
+
 __global__ void k_set_meta(int* meta, int idx, int v) { meta[idx] = v; }
 
 __global__ void k_set_int(int* p, int v) { *p = v; }
@@ -674,6 +701,20 @@ void enqueue_append(sph_system* s, int n0, int m, int ref0, int sys, const doubl
     k_append<<<nblk(m), 256, 0, s->stream>>>(n0, m, ref0, sys, in_dev, has_v, has_rho, has_P,
                                             has_type, s->cols[s->cur], s->icols[s->cur], s->cap);
     k_set_meta<<<1, 1, 0, s->stream>>>(s->meta, META_N, n0 + m);
+}
+
+static_assert(CNT_COPIES == 64, "k_report sums one copy per lane");
+
+void enqueue_report(sph_system* s)
+{
+    k_report<<<1, 256, 0, s->stream>>>(s->meta, s->mask_total, s->pair_counter, s->sys_cnt,
+                                       (int)s->sys_host.size(), s->report, s->sys_cnt_host);
+}
+
+// The descriptor of system `slot` as the host has it now.
+void enqueue_set_sys(sph_system* s, int slot)
+{
+    k_set_sys<<<1, 64, 0, s->stream>>>(s->sysd + slot, s->sys_host[slot]);
 }
 
 void enqueue_set_int(sph_system* s, int* p, int v) { k_set_int<<<1, 1, 0, s->stream>>>(p, v); }
