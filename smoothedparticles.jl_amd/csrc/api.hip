@@ -709,7 +709,7 @@ int run_pair(sph_system* s, int op, int self, int overwrite, unsigned long long*
         queue_set = 0;
     }
     s->queue_used |= 1u << queue_set;
-    c.queue += queue_set * NQUEUE * QSTRIDE;
+    c.queue += queue_set * QSET;
     c.loading = loading;
     launch_pair(op, s->precision, s->rows, s->flat, s->periodic, c, pair_grid(ntiles), s->stream);
     prof_end(s, prof_kernel, ev);
@@ -762,7 +762,7 @@ int new_handle(int precision, sph_system** out)
         rc = fail(SPH_EHIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
     }
     if (!rc && !(rc = dalloc(s, &s->meta, META_SLOTS)) && !(rc = dalloc(s, &s->pair_counter, CNT_SLOTS)) &&
-        !(rc = dalloc(s, &s->queue, NQUEUE_SETS * NQUEUE * QSTRIDE)) &&
+        !(rc = dalloc(s, &s->queue, NQUEUE_SETS * QSET)) &&
         !(rc = dalloc(s, &s->mask_total, 1))) {
         e = hipHostMalloc((void**)&s->report, sizeof(Report), hipHostMallocDefault);
         if (e != hipSuccess) {
@@ -796,7 +796,7 @@ int destroy(sph_system* s)
     free_particle_arrays(s);
     free_cell_arrays(s);
     dfree(s, s->meta, META_SLOTS); dfree(s, s->pair_counter, CNT_SLOTS);
-    dfree(s, s->queue, NQUEUE_SETS * NQUEUE * QSTRIDE);
+    dfree(s, s->queue, NQUEUE_SETS * QSET);
     dfree(s, s->masks, s->mask_cap); dfree(s, s->mask_total, 1);
     dfree(s, s->kept, s->kept_cap); dfree(s, s->kept_rg, s->kept_cap);
     dfree(s, s->sysd, s->sysd_cap); dfree(s, s->sys_cnt, SYSCNT * s->sys_cnt_cap);
@@ -1638,7 +1638,7 @@ int autotune(sph_system* s, int* best)
 namespace sph {
 __global__ void k_reset_queue(int* queue)
 {
-    if (threadIdx.x < NQUEUE) queue[threadIdx.x * QSTRIDE] = 0;
+    if (threadIdx.x <= NQUEUE) queue[threadIdx.x * QSTRIDE] = 0;
 }
 // Clears queue set 0, for a pass about to use it.
 void reset_queue(sph_system* s)

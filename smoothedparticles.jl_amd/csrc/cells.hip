@@ -464,7 +464,7 @@ __global__ __launch_bounds__(256) void k_tile_table(
     if (threadIdx.x == 0) with_tiles = 0;
     const int b = chain_ticket(ticket);  // (a block barrier)
     if (b == 0) {
-        if (threadIdx.x < NQUEUE * NQUEUE_SETS) queue[threadIdx.x * QSTRIDE] = 0;
+        if (threadIdx.x < NQUEUE_SETS * QSET / QSTRIDE) queue[threadIdx.x * QSTRIDE] = 0;
         if (removal && meta[META_NREM] != 0)
             for (int s = threadIdx.x; s < nsys; s += 256)
                 remove_seq(s, ncells, sc, cell_start, ref, inv);

@@ -105,9 +105,13 @@ __device__ inline void count_tests(const PairCtx& c, unsigned long long n)
 // tile behind an atomic, and every idle wave trying all heads, a pass took
 // 86 us however little it had to do (8192 waves on 8 heads; a 2D dam break of
 // 6514 particles: 13.6 -> 7.2 ms per 50 steps).  A queue whose tiles are all dealt
-// out is not touched.  (Reading another XCD's head before trying it spares
-// its last atomics but made the waves that help slower: the force pass of
-// the 5.75M-particle dam break took 3.25 instead of 3.06 ms.)
+// out is not touched, and the wave that first finds a queue empty says so in
+// the set's mask, which the others read when their queue runs out: one read
+// each instead of up to seven failing atomics (97k-particle 2D dam break with
+// T = 16, a little more than one tile per wave: 266 -> 165 us per step; 333k
+// with T = 32: 306 -> 246).  (Reading another queue's head
+// before trying it made the waves that help slower: the force pass of the
+// 5.75M-particle dam break took 3.25 instead of 3.06 ms.)
 // With one tile per grab the tiles in flight on an XCD are consecutive and
 // share their neighbour cells in the L2 (3D: 9.6 instead of 10.6 ms per
 // dam-break step); the short 2D tiles take four per grab, which spares
@@ -143,20 +147,27 @@ __device__ inline void tile_cursor_init(const PairCtx& c, int ntiles, TileCursor
 __device__ inline int next_tile(const PairCtx& c, int ntiles, TileCursor& tc)
 {
     if (tc.cur < tc.end) return tc.cur++;
+    int* mask = &c.queue[NQUEUE * QSTRIDE];
+    unsigned empty = 0;
     for (; tc.k < NQUEUE; ++tc.k) {
         const int q = (int)((blockIdx.x + tc.k) % NQUEUE);
         const int dealt = queue_dealt(tc, q);
         const int lo = queue_lo(ntiles, q) + dealt, hi = queue_lo(ntiles, q + 1);
-        if (lo >= hi) continue;
-        int* head = &c.queue[q * QSTRIDE];
+        if (lo >= hi || ((empty >> q) & 1u)) continue;
         int start = 0;
-        if (__lane_id() == 0) start = atomicAdd(head, c.qgrab);
+        if (__lane_id() == 0) start = atomicAdd(&c.queue[q * QSTRIDE], c.qgrab);
         start = __builtin_amdgcn_readfirstlane(start);
         if (start < hi - lo) {
             tc.cur = lo + start;
             tc.end = min(hi, lo + start + c.qgrab);
             return tc.cur++;
         }
+        int seen = 0;
+        if (__lane_id() == 0) {
+            if (start < hi - lo + c.qgrab) atomicOr(mask, 1 << q);  // the first to find it empty
+            seen = __hip_atomic_load(mask, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        empty = (unsigned)__builtin_amdgcn_readfirstlane(seen);
     }
     return ntiles;
 }

@@ -110,7 +110,7 @@ struct PairCtx {
     int masks_mixed;          // the masks were stored by a mixed-precision pass
     const int* cell_start;
     const int* meta;
-    int* queue;               // NQUEUE tile-queue heads, QSTRIDE ints apart
+    int* queue;               // a set of NQUEUE tile-queue heads, QSTRIDE ints apart
     int qgrab;                // tiles taken per queue atomic
     double* cols;             // current column buffer
     const int* refidx;
@@ -141,6 +141,8 @@ static constexpr int QSTRIDE = 32;
 // Sets of queue heads: a cell build clears them all, and the first passes
 // after it take one each (the others clear set 0 first).
 static constexpr int NQUEUE_SETS = 2;
+// A set: the heads, then a line with the mask of the queues known to be empty.
+static constexpr int QSET = (NQUEUE + 1) * QSTRIDE;
 
 // The pair passes count accepted pairs and distance tests in CNT_COPIES
 // copies of the counters, each on its own 128-byte line: a wave adds to copy
@@ -332,7 +334,7 @@ struct sph_system {
 
     int* meta;           // device counters
     sph::Report* report; // pinned
-    int* queue;          // NQUEUE_SETS * NQUEUE * QSTRIDE ints: tile-queue heads
+    int* queue;          // NQUEUE_SETS * QSET ints: tile-queue heads
     unsigned queue_used; // bit per set: used since a build cleared them
     unsigned long long* pair_counter;  // CNT_SLOTS: density pairs, force pairs, tests
 
