@@ -277,8 +277,9 @@ int sph_key_geometry(sph_system* s, int64_t* key_phase, int64_t* key_lim,
 
 /* Targets per tile of the pair kernels (8, 16, 32 or 64; 0 = automatic: the
  * smallest power of two >= the mean occupancy of the non-empty cells, at
- * most 64, chosen at each sph_build_cells).  The summation order of the
- * pair sums, hence their last bits, depends on the tile size.
+ * most 64 in SPH_MIXED mode and 32 in SPH_FP64 mode, chosen at each
+ * sph_build_cells).  The summation order
+ * of the pair sums, hence their last bits, depends on the tile size.
  * sph_autotune: in SPH_MIXED mode it times the density and force passes for
  * each tile size on the current cell list and keeps the fastest; in SPH_FP64
  * mode it keeps the automatic choice, so the plain FP64 path gives the same

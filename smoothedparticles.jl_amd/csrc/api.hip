@@ -593,10 +593,19 @@ void prof_collect(sph_system* s)
     s->ev_open.clear();
 }
 
-int choose_tile(double occupancy)
+// Targets per tile: the smallest power of two >= the mean occupancy of the
+// cells, at most 64 in the mixed mode and 32 in FP64: a tile of 32 spreads its
+// pairs over the lanes more evenly than one of 64, and the FP64 walk is what
+// costs (3D dam break, us per step at T = 64 / 32: 105k particles 674 / 468,
+// 311k 1190 / 825, 1.7M 4375 / 3970, 5.76M 14550 / 13790).  The mixed mode's
+// shorter walk gains from it only below 640k particles (105k 366 / 308, 842k
+// 1079 / 1114, 5.76M 6440 / 7540), where it would change FP32 roundings for
+// 15%; there it is left to autotuning.
+int choose_tile(double occupancy, int precision)
 {
+    const int cap = precision == SPH_MIXED ? 64 : 32;
     int T = 8;
-    while (T < 64 && T < occupancy) T <<= 1;
+    while (T < cap && T < occupancy) T <<= 1;
     return T;
 }
 
@@ -968,7 +977,8 @@ int build_cells(sph_system* s)
     HIPC(hipGetLastError());
     if ((rc = sync_meta(s))) return rc;
     if (s->tile_auto && s->report->meta[META_NCELLS] > 0) {
-        const int T = choose_tile((double)s->n / s->report->meta[META_NCELLS]);
+        const int T = choose_tile((double)s->n / s->report->meta[META_NCELLS],
+                                  s->precision);
         if (T != s->tile_T) {
             s->tile_T = T;
             enqueue_tiles(s);
@@ -1569,7 +1579,8 @@ int autotune(sph_system* s, int* best)
         // input gives the same bits on every run.
         int rc = sph_set_tile(s, 0);
         if (!rc && s->report->meta[META_NCELLS] > 0) {
-            const int T = choose_tile((double)s->n / s->report->meta[META_NCELLS]);
+            const int T = choose_tile((double)s->n / s->report->meta[META_NCELLS],
+                                  s->precision);
             rc = sph_set_tile(s, T);
             if (!rc) rc = sph_set_tile(s, 0);
         }
