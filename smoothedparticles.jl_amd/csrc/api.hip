@@ -49,7 +49,7 @@ void enqueue_lattice_write(sph_system* s, const LatticeGeo& g, const sph_lattice
                            const unsigned* flags, const unsigned* pos, long long nlat, int slot,
                            int ref0);
 void enqueue_report(sph_system* s);
-void enqueue_set_sys(sph_system* s, int slot);
+void enqueue_params0(sph_system* s);
 void enqueue_fill_int(sph_system* s, int* p, int v, long long n);
 void enqueue_remap_sys(sph_system* s, const int* map_dev);
 long long scan_partials_needed(long long n);
@@ -538,6 +538,7 @@ int upload_sysd(sph_system* s)
         HIPC(hipMemcpyAsync(s->sysd, s->sys_host.data(), sizeof(SysDesc) * n,
                             hipMemcpyHostToDevice, s->stream));
     HIPC(hipStreamSynchronize(s->stream));
+    s->params0_stale = false;
     return 0;
 }
 
@@ -709,6 +710,7 @@ int run_pair(sph_system* s, int op, int self, int overwrite, unsigned long long*
     c.test_counter = tests;
     c.mask_mode = s->use_masks ? mask_mode : MASK_TEST;
     c.only_flagged = only_flagged;
+    enqueue_params0(s);
     hipEvent_t ev[2];
     prof_begin(s, ev);
     for (int q = 0; q < NQUEUE_SETS && queue_set < 0; ++q)
@@ -993,12 +995,15 @@ int build_cells(sph_system* s)
     return 0;
 }
 
-// Single-system calls carry their parameters: they become slot 0's.
+// Single-system calls carry their parameters: they become slot 0's, on the
+// device when a pair pass, a fused step or a reduction needs them there.
 int set_params0(sph_system* s, const sph_params* p)
 {
     if (nsys(s) == 0) return fail(SPH_ESTATE, "the handle holds no system");
-    s->sys_host[0].ph = make_phys(s->sys_host[0].g, p);
-    enqueue_set_sys(s, 0);  // by value: the host table may change again at once
+    const Phys ph = make_phys(s->sys_host[0].g, p);
+    if (std::memcmp(&ph, &s->sys_host[0].ph, sizeof(Phys)) == 0) return 0;
+    s->sys_host[0].ph = ph;
+    s->params0_stale = true;  // uploaded before the first kernel that reads it
     return 0;
 }
 
@@ -1119,6 +1124,7 @@ int run_steps(sph_system* s, int scheme, int nsteps)
         s->step_pairs[0] = s->step_pairs[1] = s->step_pairs[2] = 0;
         return 0;
     }
+    enqueue_params0(s);
     // Tiles are taken from a work queue: the grid needs no tile count.
     const long long tiles_bound = s->tile_cap;
     if ((rc = clear_counters(s))) return rc;
@@ -1269,8 +1275,7 @@ int reduce_slot(sph_system* s, int slot, int what, double* out)
 }
 
 // Probe sums of system `slot` (SmoothedParticles.sum at points,
-// src/core.jl:240-258).  The probe and result staging is allocated per call:
-// the call runs at frame cadence, not in the step loop.
+// src/core.jl:240-258).
 int probe_sum(sph_system* s, int slot, double m, int flags, const double* x, long long np,
               double* out)
 {
@@ -1280,8 +1285,11 @@ int probe_sum(sph_system* s, int slot, double m, int flags, const double* x, lon
         return fail(SPH_EUNSUP, "probe sums of periodic systems are not supported");
     if (!s->cells_valid) return fail(SPH_ESTATE, "cell list is not current");
     if (np == 0) return 0;
-    double* buf = nullptr;
-    HIPC(hipMalloc((void**)&buf, sizeof(double) * 7 * (size_t)np));
+    // the field-transfer buffer holds points and sums unless there are more of
+    // them than it has room for
+    const bool own = 7 * np > 9 * s->cap;
+    double* buf = s->stage;
+    if (own) HIPC(hipMalloc((void**)&buf, sizeof(double) * 7 * (size_t)np));
     double* pin = buf;
     double* pout = buf + 3 * np;
     hipError_t e = hipMemcpyAsync(pin, x, sizeof(double) * 3 * np, hipMemcpyHostToDevice, s->stream);
@@ -1289,11 +1297,12 @@ int probe_sum(sph_system* s, int slot, double m, int flags, const double* x, lon
         enqueue_probe_sum(s, slot, pin, np, m, (flags & SPH_PROBE_FLUID_ONLY) ? 1 : 0, pout);
         e = hipGetLastError();
     }
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(out, pout, sizeof(double) * 4 * np, hipMemcpyDeviceToHost, s->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    const hipError_t ef = hipFree(buf);
+    int rc = 0;
+    if (e == hipSuccess) rc = download(s, out, pout, sizeof(double) * 4 * (size_t)np);
+    else (void)hipStreamSynchronize(s->stream);
+    const hipError_t ef = own ? hipFree(buf) : hipSuccess;
     if (e != hipSuccess) return fail(SPH_EHIP, std::string("probe sum: ") + hipGetErrorString(e));
+    if (rc) return rc;
     if (ef != hipSuccess) return fail(SPH_EHIP, std::string("hipFree: ") + hipGetErrorString(ef));
     return 0;
 }

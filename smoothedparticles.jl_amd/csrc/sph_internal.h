@@ -320,6 +320,7 @@ struct sph_system {
     std::vector<long long> sys_n;      // particles per system (host mirror)
     std::vector<long long> sys_off;    // first particle of each system (valid with cells)
     sph::SysDesc* sysd;                // device copy
+    bool params0_stale;                // sys_host[0].ph is newer than the device's
     long long sysd_cap;
     int* cell_sys;                     // global cell -> system
     long long cells_total;             // sum of key_max of all systems

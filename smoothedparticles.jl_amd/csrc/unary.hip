@@ -12,14 +12,18 @@ namespace sph {
 #define UCOL(cols, cap, f, i) ((cols)[(long long)(f) * (cap) + (i)])
 
 // ------------------------------------------------------------ operators --
+// A handle of one system passes its parameters by value (one != 0): the
+// operators of a program's loop come with different parameters call by call,
+// and an upload of its own cost each call a launch.
 __global__ __launch_bounds__(256) void k_unary(int op, const int* meta, double* cols,
                                                long long cap, const SysDesc* __restrict__ sysd,
-                                               const int* __restrict__ sysid, double* prho2)
+                                               const int* __restrict__ sysid, double* prho2,
+                                               int one, Phys ph1)
 {
     const int n = meta[META_N];
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const Phys& ph = sysd[sysid[i]].ph;
+    const Phys ph = one ? ph1 : sysd[sysid[i]].ph;
     switch (op) {
     case SPH_OP_RESET_RHO:  // tests/test_collision_2d.jl:84-86
         UCOL(cols, cap, C_RHO, i) = 0.0;
@@ -607,13 +611,17 @@ __global__ __launch_bounds__(256) void k_fill_int(int* p, int v, long long n)
 // ------------------------------------------------------------ launchers --
 static inline unsigned nblk(long long n) { return (unsigned)((n + 255) / 256); }
 
+void enqueue_params0(sph_system* s);
+
 static inline const int* sysid_col(sph_system* s) { return s->icols[s->cur] + I_SYS * s->cap; }
 
 void enqueue_unary(sph_system* s, int op, double* prho2)
 {
     if (s->n <= 0) return;
+    const int one = s->sys_host.size() == 1;
     k_unary<<<nblk(s->n), 256, 0, s->stream>>>(op, s->meta, s->cols[s->cur], s->cap, s->sysd,
-                                              sysid_col(s), prho2);
+                                              sysid_col(s), prho2, one,
+                                              one ? s->sys_host[0].ph : Phys{});
 }
 
 void enqueue_prho2(sph_system* s)
@@ -641,6 +649,7 @@ long long reduce_partials_needed(long long n) { return (n + 256 * RED_ITEMS - 1)
 void enqueue_reduce(sph_system* s, int sys, long long off, long long n, int what, double* out_dev)
 {
     const int nb = (int)((n + 256 * RED_ITEMS - 1) / (256 * RED_ITEMS));
+    enqueue_params0(s);
     if (nb > 0)
         k_reduce_part<<<nb, 256, 0, s->stream>>>(what, (int)off, (int)n, s->cols[s->cur], s->cap,
                                                  s->sysd, sys, s->red_part);
@@ -711,10 +720,13 @@ void enqueue_report(sph_system* s)
                                        (int)s->sys_host.size(), s->report, s->sys_cnt_host);
 }
 
-// The descriptor of system `slot` as the host has it now.
-void enqueue_set_sys(sph_system* s, int slot)
+// The parameters of slot 0 as the host has them now, if the device's copy is
+// older.
+void enqueue_params0(sph_system* s)
 {
-    k_set_sys<<<1, 64, 0, s->stream>>>(s->sysd + slot, s->sys_host[slot]);
+    if (!s->params0_stale) return;
+    k_set_sys<<<1, 64, 0, s->stream>>>(s->sysd, s->sys_host[0]);
+    s->params0_stale = false;
 }
 
 void enqueue_set_int(sph_system* s, int* p, int v) { k_set_int<<<1, 1, 0, s->stream>>>(p, v); }
