@@ -22,7 +22,7 @@
 using namespace sph;
 
 namespace sph {
-void enqueue_build(sph_system* s, unsigned skip_cols = 0, int skip_a = 0);
+void enqueue_build(sph_system* s, unsigned skip_cols = 0, int skip_a = 0, int kick = 0);
 void enqueue_tiles(sph_system* s);
 void enqueue_unary(sph_system* s, int op, double* prho2);
 void enqueue_prho2(sph_system* s);
@@ -1043,8 +1043,9 @@ int cd_step(sph_system* s, long long tiles_bound)
 }
 
 // One step of a density-summation scheme: build; density pass (stores the
-// masks); EOS with P/rho^2; force pass (loads them); kick and drift.
-int ds_step(sph_system* s, int eos, long long tiles_bound)
+// masks); EOS with P/rho^2; force pass (loads them); kick and drift -- by the
+// next step's build, except after the last step of a call (or of a graph).
+int ds_step(sph_system* s, int eos, long long tiles_bound, bool first, bool last)
 {
     int rc;
     hipEvent_t ev[2];
@@ -1053,7 +1054,7 @@ int ds_step(sph_system* s, int eos, long long tiles_bound)
     // EOS then P of every particle, before anything reads them: the build
     // need not carry the two columns over, nor the acceleration of the fluid,
     // which the force pass overwrites
-    enqueue_build(s, (1u << C_RHO) | (1u << C_P), 1);
+    enqueue_build(s, (1u << C_RHO) | (1u << C_P), 1, !first);
     prof_end(s, SPH_KERNEL_BUILD, ev);
     if ((rc = run_pair(s, P_DENSITY, 1, 1, s->pair_counter, tiles_bound, SPH_KERNEL_DENSITY,
                        MASK_TEST_STORE, 0, s->pair_counter + 2, 0)))
@@ -1064,17 +1065,20 @@ int ds_step(sph_system* s, int eos, long long tiles_bound)
     if ((rc = run_pair(s, P_FORCE, 0, 1, s->pair_counter + 1, tiles_bound, SPH_KERNEL_FORCE,
                        MASK_LOAD, 0, nullptr, 1)))
         return rc;
-    prof_begin(s, ev);
-    enqueue_kick_drift(s);
-    prof_end(s, SPH_KERNEL_UNARY, ev);
+    if (last) {
+        prof_begin(s, ev);
+        enqueue_kick_drift(s);
+        prof_end(s, SPH_KERNEL_UNARY, ev);
+    }
     HIPC(hipGetLastError());
     return 0;
 }
 
-int one_step(sph_system* s, int scheme, int eos, long long tiles_bound)
+// first, last: the step's place in the call (or in the graph).
+int one_step(sph_system* s, int scheme, int eos, long long tiles_bound, bool first, bool last)
 {
     return scheme == SPH_SCHEME_COLLAPSE_DRY ? cd_step(s, tiles_bound)
-                                             : ds_step(s, eos, tiles_bound);
+                                             : ds_step(s, eos, tiles_bound, first, last);
 }
 
 // With SPH_OPTION_GRAPH the steps of a call are replayed from a hipGraph:
@@ -1096,7 +1100,8 @@ int run_graph(sph_system* s, int scheme, int eos, long long tiles_bound, int per
         s->prof = prof;
         return fail(SPH_EHIP, std::string("hipStreamBeginCapture: ") + hipGetErrorString(e));
     }
-    for (int k = 0; k < per && !rc; ++k) rc = one_step(s, scheme, eos, tiles_bound);
+    for (int k = 0; k < per && !rc; ++k)
+        rc = one_step(s, scheme, eos, tiles_bound, k == 0, k == per - 1);
     e = hipStreamEndCapture(s->stream, &graph);
     s->prof = prof;
     if (rc) {
@@ -1134,8 +1139,8 @@ int run_steps(sph_system* s, int scheme, int nsteps)
         if ((rc = run_graph(s, scheme, eos, tiles_bound, per, nsteps / per))) return rc;
         k = nsteps / per * per;
     }
-    for (; k < nsteps; ++k)
-        if ((rc = one_step(s, scheme, eos, tiles_bound))) return rc;
+    for (const int k0 = k; k < nsteps; ++k)
+        if ((rc = one_step(s, scheme, eos, tiles_bound, k == k0, k == nsteps - 1))) return rc;
     if ((rc = sync_meta(s))) return rc;
     for (int i = 0; i < 3; ++i) s->step_pairs[i] = s->report->pairs[i];
     if (nsteps > 0) {
