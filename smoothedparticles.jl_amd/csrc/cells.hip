@@ -474,9 +474,11 @@ __device__ inline int cell_chunks(const SysDesc& d, const int* cell_start, int l
 // cell_start[c] + k*T ...; its pair masks start at the mask words of the
 // tiles before it (chunks * T words each), its kept-candidate list at 64 / T
 // times that.  Each thread takes TT_CELLS consecutive ranks; tiles and mask
-// words are scanned together, by two waves of each block (chained blocks).
-// The first block also clears the tile queues and replays the removals.
-static constexpr int TT_CELLS = 4;
+// words are scanned together, by two waves of each block (chained blocks).  One
+// cell per thread: a small grid's table waits on one cell's loads and divisions
+// (1.5k cells 10.5 -> 7.0 us against four), a large one's chain is longer (93k
+// cells 24 -> 31 us of a 6.4 ms step).  The first block also clears the tile queues and replays the removals.
+static constexpr int TT_CELLS = 1;
 static constexpr int TT_TILE = 256 * TT_CELLS;
 
 template <int ROWS>
