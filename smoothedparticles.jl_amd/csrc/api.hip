@@ -24,7 +24,7 @@ using namespace sph;
 namespace sph {
 void enqueue_build(sph_system* s, unsigned skip_cols = 0, int skip_a = 0, int kick = 0);
 void enqueue_tiles(sph_system* s);
-void enqueue_unary(sph_system* s, int op, double* prho2);
+void enqueue_unary(sph_system* s, int op);
 void enqueue_prho2(sph_system* s);
 void enqueue_kick_drift(sph_system* s);
 void enqueue_cd_unary(sph_system* s, int stage);
@@ -625,6 +625,7 @@ PairCtx make_ctx(sph_system* s)
     c.cols = s->cols[s->cur];
     c.refidx = s->icols[s->cur] + I_REF * s->cap;
     c.prho2 = s->prho2;
+    c.prho2_out = s->prho2;
     c.masks = s->masks;
     c.kept = s->use_kept ? s->kept : nullptr;
     c.kept_rg = s->kept_rg;
@@ -701,7 +702,8 @@ int pair_grid(long long ntiles)
 // cleared again.
 int run_pair(sph_system* s, int op, int self, int overwrite, unsigned long long* counter,
              long long ntiles, int prof_kernel, int mask_mode, int only_flagged = 0,
-             unsigned long long* tests = nullptr, int queue_set = -1, int loading = LOAD_ASK)
+             unsigned long long* tests = nullptr, int queue_set = -1, int loading = LOAD_ASK,
+             int eos = EOS_NONE)
 {
     PairCtx c = make_ctx(s);
     c.self = self;
@@ -722,6 +724,7 @@ int run_pair(sph_system* s, int op, int self, int overwrite, unsigned long long*
     s->queue_used |= 1u << queue_set;
     c.queue += queue_set * QSET;
     c.loading = loading;
+    c.eos = eos;
     launch_pair(op, s->precision, s->rows, s->flat, s->periodic, c, pair_grid(ntiles), s->stream);
     prof_end(s, prof_kernel, ev);
     HIPC(hipGetLastError());
@@ -1025,7 +1028,7 @@ int cd_step(sph_system* s, long long tiles_bound)
                        MASK_TEST, 0, s->pair_counter + 2, 0)))
         return rc;
     prof_begin(s, ev);
-    enqueue_unary(s, SPH_OP_FIND_PRESSURE_CONTINUITY, nullptr);
+    enqueue_unary(s, SPH_OP_FIND_PRESSURE_CONTINUITY);
     enqueue_cd_unary(s, CD_MOVE);
     prof_end(s, SPH_KERNEL_UNARY, ev);
     prof_begin(s, ev);
@@ -1043,7 +1046,7 @@ int cd_step(sph_system* s, long long tiles_bound)
 }
 
 // One step of a density-summation scheme: build; density pass (stores the
-// masks); EOS with P/rho^2; force pass (loads them); kick and drift -- by the
+// masks, and applies the EOS where it writes rho); force pass (loads them); kick and drift -- by the
 // next step's build, except after the last step of a call (or of a graph).
 int ds_step(sph_system* s, int eos, long long tiles_bound, bool first, bool last)
 {
@@ -1057,11 +1060,8 @@ int ds_step(sph_system* s, int eos, long long tiles_bound, bool first, bool last
     enqueue_build(s, (1u << C_RHO) | (1u << C_P), 1, !first);
     prof_end(s, SPH_KERNEL_BUILD, ev);
     if ((rc = run_pair(s, P_DENSITY, 1, 1, s->pair_counter, tiles_bound, SPH_KERNEL_DENSITY,
-                       MASK_TEST_STORE, 0, s->pair_counter + 2, 0)))
+                       MASK_TEST_STORE, 0, s->pair_counter + 2, 0, LOAD_ASK, eos)))
         return rc;
-    prof_begin(s, ev);
-    enqueue_unary(s, eos, s->prho2);
-    prof_end(s, SPH_KERNEL_UNARY, ev);
     if ((rc = run_pair(s, P_FORCE, 0, 1, s->pair_counter + 1, tiles_bound, SPH_KERNEL_FORCE,
                        MASK_LOAD, 0, nullptr, 1)))
         return rc;
@@ -1123,7 +1123,7 @@ int run_steps(sph_system* s, int scheme, int nsteps)
         scheme != SPH_SCHEME_COLLAPSE_DRY)
         return fail(SPH_EUNSUP, "unknown scheme");
     if (nsteps < 0) return fail(SPH_EINVAL, "negative step count");
-    const int eos = scheme == SPH_SCHEME_WCSPH_SE ? SPH_OP_FIND_PRESSURE : SPH_OP_FIND_PRESSURE_RHO0;
+    const int eos = scheme == SPH_SCHEME_WCSPH_SE ? EOS_RHO0 : EOS_RHO0_FIELD;
     int rc;
     if (nsys(s) == 0) {
         s->step_pairs[0] = s->step_pairs[1] = s->step_pairs[2] = 0;
@@ -1791,7 +1791,7 @@ int sph_apply_unary(sph_system* s, int op, const sph_params* params)
     if (rc) return rc;
     hipEvent_t ev[2];
     prof_begin(s, ev);
-    enqueue_unary(s, op, nullptr);
+    enqueue_unary(s, op);
     prof_end(s, SPH_KERNEL_UNARY, ev);
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(s->stream));

@@ -45,6 +45,14 @@ namespace sph {
 __device__ inline void sys_prep(int nsys, int* sc, int* meta)
 {
     __shared__ int part[4];
+    if (threadIdx.x == 0) meta[META_NTOT] = meta[META_N];
+    if (nsys == 1) {  // nothing to scan, no barrier
+        if (threadIdx.x == 0) {
+            sc[SC_NTOT] = sc[SC_N];
+            sc[SC_REFBASE] = 0;
+        }
+        return;
+    }
     int carry = 0;
     for (int s0 = 0; s0 < nsys; s0 += 256) {
         const int s = s0 + (int)threadIdx.x;
@@ -68,7 +76,6 @@ __device__ inline void sys_prep(int nsys, int* sc, int* meta)
         carry += round;
         __syncthreads();
     }
-    if (threadIdx.x == 0) meta[META_NTOT] = meta[META_N];
 }
 
 // ------------------------------------------------------------------ keys --

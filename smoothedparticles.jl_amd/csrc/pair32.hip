@@ -103,6 +103,7 @@ struct Density32 {
         v = v + d.ph.kW * w;
         if (c.self) v = v + d.ph.kW;
         COL(c, out_col, p) = v;
+        write_eos(c, d, p, v);
     }
 };
 

@@ -117,6 +117,7 @@ struct Density64 {
         v = v + d.ph.kW * a.w;
         if (c.self) v = v + d.ph.kW;
         COL(c, OUT, p) = v;
+        if constexpr (OUT == C_RHO) write_eos(c, d, p, v);
     }
 };
 

@@ -945,6 +945,20 @@ __device__ inline void digest_write(const PairCtx& c, int p, unsigned long long 
     c.pair_out[2 * r + 1] = (long long)h;
 }
 
+// ------------------------------------------------------------------- EOS --
+// The equation of state of particle p whose density rho the pass has just
+// formed: the expressions of SPH_OP_FIND_PRESSURE(_RHO0).  A kernel of its own
+// that read rho back took 43 us of a 5.75M-particle step and 4 of a small one's
+// 75; here it costs nothing measurable (the density kernel has no spills).
+__device__ inline void write_eos(const PairCtx& c, const SysDesc& d, int p, double rho)
+{
+    if (c.eos == EOS_NONE) return;
+    const double rho0 = c.eos == EOS_RHO0_FIELD ? COL(c, C_RHO0, p) : d.ph.rho0;
+    const double P = (d.ph.c * d.ph.c) * (rho - rho0);
+    COL(c, C_P, p) = P;
+    c.prho2_out[p] = P / (rho * rho);
+}
+
 // -------------------------------------------------------------- launch --
 // Blocks of a kernel that the current device holds at once (one-wave
 // blocks, static LDS).

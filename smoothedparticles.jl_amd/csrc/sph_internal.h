@@ -115,6 +115,8 @@ struct PairCtx {
     double* cols;             // current column buffer
     const int* refidx;
     const double* prho2;      // P/rho^2 per particle (force pass)
+    int eos;                  // density pass: form P and P/rho^2 where it writes rho (EOS_*)
+    double* prho2_out;
     unsigned long long* pair_counter;  // in the first copy (CNT_COPIES), or null
     unsigned long long* test_counter;  // distance tests of a testing pass (may be null)
     unsigned long long* emit_counter;
@@ -125,6 +127,10 @@ struct PairCtx {
     int only_flagged;         // skip systems whose pass_on is 0
     int loading;              // kernels of a loading pass: LOAD_* (the device decides, or known)
 };
+
+// The equation of state a fused step's density pass applies: none,
+// P = c^2 (rho - rho0) with the system's rho0, or with the rho0 field.
+enum Eos { EOS_NONE = 0, EOS_RHO0 = 1, EOS_RHO0_FIELD = 2 };
 
 // A pass that loads the masks launches the kernel for masks with kept lists
 // and the general one, and the device's mask state picks the one that works,

@@ -17,8 +17,7 @@ namespace sph {
 // and an upload of its own cost each call a launch.
 __global__ __launch_bounds__(256) void k_unary(int op, const int* meta, double* cols,
                                                long long cap, const SysDesc* __restrict__ sysd,
-                                               const int* __restrict__ sysid, double* prho2,
-                                               int one, Phys ph1)
+                                               const int* __restrict__ sysid, int one, Phys ph1)
 {
     const int n = meta[META_N];
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -35,16 +34,12 @@ __global__ __launch_bounds__(256) void k_unary(int op, const int* meta, double* 
         break;
     case SPH_OP_FIND_PRESSURE: {  // examples/collapse_dry.jl:126
         const double rho = UCOL(cols, cap, C_RHO, i);
-        const double P = (ph.c * ph.c) * (rho - ph.rho0);
-        UCOL(cols, cap, C_P, i) = P;
-        if (prho2) prho2[i] = P / (rho * rho);
+        UCOL(cols, cap, C_P, i) = (ph.c * ph.c) * (rho - ph.rho0);
         break;
     }
     case SPH_OP_FIND_PRESSURE_RHO0: {  // tests/test_collision_2d.jl:71-73
         const double rho = UCOL(cols, cap, C_RHO, i);
-        const double P = (ph.c * ph.c) * (rho - UCOL(cols, cap, C_RHO0, i));
-        UCOL(cols, cap, C_P, i) = P;
-        if (prho2) prho2[i] = P / (rho * rho);
+        UCOL(cols, cap, C_P, i) = (ph.c * ph.c) * (rho - UCOL(cols, cap, C_RHO0, i));
         break;
     }
     case SPH_OP_FIND_PRESSURE_CONTINUITY: {  // examples/collapse_dry.jl:123-127
@@ -52,9 +47,7 @@ __global__ __launch_bounds__(256) void k_unary(int op, const int* meta, double* 
         rho = rho + UCOL(cols, cap, C_DRHO, i) * ph.dt;
         UCOL(cols, cap, C_RHO, i) = rho;
         UCOL(cols, cap, C_DRHO, i) = 0.0;
-        const double P = (ph.c * ph.c) * (rho - ph.rho0);
-        UCOL(cols, cap, C_P, i) = P;
-        if (prho2) prho2[i] = P / (rho * rho);
+        UCOL(cols, cap, C_P, i) = (ph.c * ph.c) * (rho - ph.rho0);
         break;
     }
     case SPH_OP_ACCELERATE: {  // examples/collapse_dry.jl:155-159
@@ -615,12 +608,12 @@ void enqueue_params0(sph_system* s);
 
 static inline const int* sysid_col(sph_system* s) { return s->icols[s->cur] + I_SYS * s->cap; }
 
-void enqueue_unary(sph_system* s, int op, double* prho2)
+void enqueue_unary(sph_system* s, int op)
 {
     if (s->n <= 0) return;
     const int one = s->sys_host.size() == 1;
     k_unary<<<nblk(s->n), 256, 0, s->stream>>>(op, s->meta, s->cols[s->cur], s->cap, s->sysd,
-                                              sysid_col(s), prho2, one,
+                                              sysid_col(s), one,
                                               one ? s->sys_host[0].ph : Phys{});
 }
 
