@@ -22,12 +22,13 @@
 using namespace sph;
 
 namespace sph {
-void enqueue_build(sph_system* s, unsigned skip_cols = 0, int skip_a = 0, int kick = 0);
+void enqueue_build(sph_system* s, unsigned skip_cols = 0, int skip_a = 0,
+                   int stage = STAGE_NONE, bool prho2 = false);
 void enqueue_tiles(sph_system* s);
 void enqueue_unary(sph_system* s, int op);
 void enqueue_prho2(sph_system* s);
 void enqueue_kick_drift(sph_system* s);
-void enqueue_cd_unary(sph_system* s, int stage);
+void enqueue_cd_kick(sph_system* s);
 void enqueue_reduce(sph_system* s, int sys, long long off, long long n, int what, double* out_dev);
 void enqueue_probe_sum(sph_system* s, int sys, const double* probes_dev, long long np, double m,
                        int fluid_only, double* out_dev);
@@ -1010,37 +1011,35 @@ int set_params0(sph_system* s, const sph_params* p)
     return 0;
 }
 
-// The time loop of examples/collapse_dry.jl:202-211 (see k_cd_unary):
-// accelerate! + move! (half steps); build; balance_of_mass!; continuity
-// find_pressure!; move!; build; P/rho^2 in the new order; internal_force!;
-// accelerate!.
-int cd_step(sph_system* s, long long tiles_bound)
+// The time loop of examples/collapse_dry.jl:202-211: accelerate! + move! (half
+// steps); build; balance_of_mass!; continuity find_pressure!; move!; build;
+// P/rho^2 in the new order; internal_force!; accelerate!.  The unary stages run
+// in the key passes of the two builds, P/rho^2 as the second one moves the
+// particles, and the last accelerate! with the next step's first -- except
+// after the last step of a call (or of a graph).  With kernels of their
+// own (five launches more) a step took 948 instead of 922 us at 532k particles,
+// 110 instead of 100 at 6.7k in 2D.
+int cd_step(sph_system* s, long long tiles_bound, bool first, bool last)
 {
     int rc;
     hipEvent_t ev[2];
     prof_begin(s, ev);
-    enqueue_cd_unary(s, CD_KICK_MOVE);
-    prof_end(s, SPH_KERNEL_UNARY, ev);
-    prof_begin(s, ev);
-    enqueue_build(s);
+    enqueue_build(s, 0, 0, first ? STAGE_CD_KICK_MOVE : STAGE_CD_KICK2_MOVE);
     prof_end(s, SPH_KERNEL_BUILD, ev);
     if ((rc = run_pair(s, P_CONTINUITY, 0, 0, s->pair_counter, tiles_bound, SPH_KERNEL_DENSITY,
                        MASK_TEST, 0, s->pair_counter + 2, 0)))
         return rc;
     prof_begin(s, ev);
-    enqueue_unary(s, SPH_OP_FIND_PRESSURE_CONTINUITY);
-    enqueue_cd_unary(s, CD_MOVE);
-    prof_end(s, SPH_KERNEL_UNARY, ev);
-    prof_begin(s, ev);
-    enqueue_build(s);
+    enqueue_build(s, 0, 0, STAGE_CD_EOS_MOVE, true);
     prof_end(s, SPH_KERNEL_BUILD, ev);
-    enqueue_prho2(s);  // the build permuted the particles
     if ((rc = run_pair(s, P_FORCE, 0, 0, s->pair_counter + 1, tiles_bound, SPH_KERNEL_FORCE,
                        MASK_TEST, 0, nullptr, 1)))
         return rc;
-    prof_begin(s, ev);
-    enqueue_cd_unary(s, CD_KICK);
-    prof_end(s, SPH_KERNEL_UNARY, ev);
+    if (last) {
+        prof_begin(s, ev);
+        enqueue_cd_kick(s);
+        prof_end(s, SPH_KERNEL_UNARY, ev);
+    }
     HIPC(hipGetLastError());
     return 0;
 }
@@ -1057,7 +1056,7 @@ int ds_step(sph_system* s, int eos, long long tiles_bound, bool first, bool last
     // EOS then P of every particle, before anything reads them: the build
     // need not carry the two columns over, nor the acceleration of the fluid,
     // which the force pass overwrites
-    enqueue_build(s, (1u << C_RHO) | (1u << C_P), 1, !first);
+    enqueue_build(s, (1u << C_RHO) | (1u << C_P), 1, first ? STAGE_NONE : STAGE_KICK_DRIFT);
     prof_end(s, SPH_KERNEL_BUILD, ev);
     if ((rc = run_pair(s, P_DENSITY, 1, 1, s->pair_counter, tiles_bound, SPH_KERNEL_DENSITY,
                        MASK_TEST_STORE, 0, s->pair_counter + 2, 0, LOAD_ASK, eos)))
@@ -1077,7 +1076,7 @@ int ds_step(sph_system* s, int eos, long long tiles_bound, bool first, bool last
 // first, last: the step's place in the call (or in the graph).
 int one_step(sph_system* s, int scheme, int eos, long long tiles_bound, bool first, bool last)
 {
-    return scheme == SPH_SCHEME_COLLAPSE_DRY ? cd_step(s, tiles_bound)
+    return scheme == SPH_SCHEME_COLLAPSE_DRY ? cd_step(s, tiles_bound, first, last)
                                              : ds_step(s, eos, tiles_bound, first, last);
 }
 

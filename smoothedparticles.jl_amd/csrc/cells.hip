@@ -122,25 +122,55 @@ __device__ inline int key_of(const SysDesc& d, int s, int nsys, int cells_total,
     return d.cell_base + (int)(ci + (long long)g.L1 * (cj + (long long)g.L2 * ck));
 }
 
-// The kick and drift that end a density-summation step (k_kick_drift) of
-// particle i: v += dt (a + g), x += dt v for fluid.
-__device__ inline void kick_drift(const Phys& ph, double* cols, long long cap, int i, double* p)
+// What a fused step leaves to the key pass of its next build, on particle i
+// at position p (KeyStage): the expressions and the order of k_kick_drift,
+// k_cd_kick and k_unary, so the bits of the operators.  STAGE_CD_KICK2_MOVE is
+// the kick that ends one collapse_dry step and the kick and move that begin
+// the next.
+__device__ inline void key_stage(int stage, const Phys& ph, double* cols, long long cap, int i,
+                                 double* p)
 {
-    if (cols[C_TYPE * cap + i] != 0.0) return;
-    const double k = ph.coeff * ph.dt;
+    const bool fluid = cols[C_TYPE * cap + i] == 0.0;
+    if (stage == STAGE_KICK_DRIFT) {  // v += dt (a + g), x += dt v
+        if (!fluid) return;
+        const double k = ph.coeff * ph.dt;
+        for (int d = 0; d < 3; ++d) {
+            const double v = cols[(C_VX + d) * cap + i] + k * (cols[(C_AX + d) * cap + i] + ph.g[d]);
+            cols[(C_VX + d) * cap + i] = v;
+            p[d] = p[d] + k * v;
+            cols[(C_X + d) * cap + i] = p[d];
+        }
+        return;
+    }
+    const double k = 0.5 * ph.dt;
+    if (stage == STAGE_CD_EOS_MOVE) {
+        double rho = cols[C_RHO * cap + i];
+        rho = rho + cols[C_DRHO * cap + i] * ph.dt;
+        cols[C_RHO * cap + i] = rho;
+        cols[C_DRHO * cap + i] = 0.0;
+        cols[C_P * cap + i] = (ph.c * ph.c) * (rho - ph.rho0);
+    }
     for (int d = 0; d < 3; ++d) {
-        const double v = cols[(C_VX + d) * cap + i] + k * (cols[(C_AX + d) * cap + i] + ph.g[d]);
-        cols[(C_VX + d) * cap + i] = v;
-        p[d] = p[d] + k * v;
-        cols[(C_X + d) * cap + i] = p[d];
+        if (fluid) {
+            double v = cols[(C_VX + d) * cap + i];
+            if (stage != STAGE_CD_EOS_MOVE) {
+                const double a = cols[(C_AX + d) * cap + i] + ph.g[d];
+                v = v + k * a;
+                if (stage == STAGE_CD_KICK2_MOVE) v = v + k * a;
+                cols[(C_VX + d) * cap + i] = v;
+            }
+            p[d] = p[d] + k * v;
+            cols[(C_X + d) * cap + i] = p[d];
+        }
+        cols[(C_AX + d) * cap + i] = 0.0;
     }
 }
 
-// KICK: first the kick and drift of the step before (one launch and one read
-// and write of the positions fewer than a kernel of its own: 5.75M particles
-// 90 + 57 us apart, 111 us together).
-template <bool KICK>
-__global__ __launch_bounds__(256) void k_keys(const SysDesc* __restrict__ sysd, int nsys,
+// With a stage, one launch and one read and write of the positions fewer than
+// a kernel of its own (5.75M particles, kick and keys: 90 + 57 us apart,
+// 111 us together).
+template <bool STAGED>
+__global__ __launch_bounds__(256) void k_keys(int stage, const SysDesc* __restrict__ sysd, int nsys,
                                               int cells_total, double* cols, long long cap,
                                               const int* __restrict__ sysid, int* meta,
                                               int* __restrict__ key, int* __restrict__ slot,
@@ -166,11 +196,11 @@ __global__ __launch_bounds__(256) void k_keys(const SysDesc* __restrict__ sysd, 
     }
     if (__all(i >= n || s == s0)) {
         if (i < n) {
-            if (KICK) kick_drift(sysd[s0].ph, cols, cap, i, p);
+            if (STAGED) key_stage(stage, sysd[s0].ph, cols, cap, i, p);
             k = key_of(sysd[s0], s0, nsys, cells_total, p[0], p[1], p[2], x, y, z, i);
         }
     } else if (i < n) {
-        if (KICK) kick_drift(sysd[s].ph, cols, cap, i, p);
+        if (STAGED) key_stage(stage, sysd[s].ph, cols, cap, i, p);
         k = key_of(sysd[s], s, nsys, cells_total, p[0], p[1], p[2], x, y, z, i);
     }
     if (i < n) key[i] = k;
@@ -288,6 +318,7 @@ struct Move {
     int skip_a;        // leave out the acceleration of fluid particles
     const int* sc;     // per-system counters (reference-index base)
     int* inv;
+    double* prho2;     // P/rho^2 in the new order, or null
 };
 
 // Particle j of the old order, with reference index r, to slot k of the new
@@ -305,6 +336,10 @@ __device__ inline void move_particle(const Move& mv, int j, int key, int r, int 
         mv.dst[C_AX * mv.cap + k] = mv.src[C_AX * mv.cap + j];
         mv.dst[C_AY * mv.cap + k] = mv.src[C_AY * mv.cap + j];
         mv.dst[C_AZ * mv.cap + k] = mv.src[C_AZ * mv.cap + j];
+    }
+    if (mv.prho2) {
+        const double rho = mv.src[C_RHO * mv.cap + j];
+        mv.prho2[k] = mv.src[C_P * mv.cap + j] / (rho * rho);
     }
     const int s = mv.isrc[I_SYS * mv.cap + j];
     mv.idst[I_REF * mv.cap + k] = r;
@@ -609,9 +644,10 @@ void enqueue_tiles(sph_system* s)
 
 // skip_cols: columns (bit C_*) the caller rewrites for every particle before
 // reading them (skip_a: the acceleration of every fluid particle); they are
-// not moved, and their values in the new order are undefined.  kick: kick and
-// drift first, as the density-summation step before left it to this build.
-void enqueue_build(sph_system* s, unsigned skip_cols, int skip_a, int kick)
+// not moved, and their values in the new order are undefined.  stage: what the
+// step before left to this build's key pass (KeyStage).  prho2: also form
+// P/rho^2 in the new order.
+void enqueue_build(sph_system* s, unsigned skip_cols, int skip_a, int stage, bool prho2)
 {
     hipStream_t st = s->stream;
     const long long cap = s->cap;
@@ -623,8 +659,8 @@ void enqueue_build(sph_system* s, unsigned skip_cols, int skip_a, int kick)
     double* c = s->cols[s->cur];
     int* ic = s->icols[s->cur];
     unsigned long long* stat = s->scan_state;
-    auto keys = kick ? k_keys<true> : k_keys<false>;
-    keys<<<nb, 256, 0, st>>>(s->sysd, nsys, ncells, c, cap, ic + I_SYS * cap, s->meta,
+    auto keys = stage != STAGE_NONE ? k_keys<true> : k_keys<false>;
+    keys<<<nb, 256, 0, st>>>(stage, s->sysd, nsys, ncells, c, cap, ic + I_SYS * cap, s->meta,
                              ic + I_KEY * cap, s->slot, s->cnt, s->sys_cnt, stat,
                              (int)scan_state_needed(s->cells_cap));
     k_scan_counts<<<nblocks(nbuckets + 1, CSCAN_TILE), 256, 0, st>>>(s->cnt, nbuckets, s->cell_start,
@@ -632,7 +668,7 @@ void enqueue_build(sph_system* s, unsigned skip_cols, int skip_a, int kick)
     k_scatter<<<nb, 256, 0, st>>>(s->meta, ic + I_KEY * cap, s->slot, ic + I_REF * cap,
                                   s->cell_start, s->tmp_idx, s->tmp_key, s->tmp_ref);
     const Move mv{c, s->cols[s->cur ^ 1], ic, s->icols[s->cur ^ 1], cap, skip_cols, skip_a,
-                  s->sys_cnt, s->inv};
+                  s->sys_cnt, s->inv, prho2 ? s->prho2 : nullptr};
     k_place<<<nb, 256, 0, st>>>(s->sysd, nsys, ncells, s->sys_cnt, s->meta, s->cell_start,
                                 s->tmp_idx, s->tmp_key, s->tmp_ref, mv);
     s->cur ^= 1;

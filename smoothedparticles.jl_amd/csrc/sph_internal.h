@@ -180,8 +180,14 @@ struct LatticeGeo {
     long long r0[3], ext[3];      // covering index range: first index and extent per axis
 };
 
-// Unary stages of the collapse_dry time loop (k_cd_unary).
-enum CdStage { CD_KICK_MOVE = 0, CD_MOVE = 1, CD_KICK = 2 };
+// What a fused step leaves to the key pass of its next build (key_stage).
+enum KeyStage {
+    STAGE_NONE = 0,
+    STAGE_KICK_DRIFT,     // end of a density-summation step
+    STAGE_CD_KICK_MOVE,   // collapse_dry: accelerate!, move!
+    STAGE_CD_KICK2_MOVE,  // the accelerate! of the step before, then accelerate!, move!
+    STAGE_CD_EOS_MOVE     // find_pressure! (continuity), move!
+};
 
 // One contiguous candidate range of a stencil row, with the periodic image
 // shift added to the candidates' coordinates.

@@ -118,36 +118,22 @@ __global__ __launch_bounds__(256) void k_kick_drift(const int* meta, double* col
     }
 }
 
-// The unary stages of the time loop of examples/collapse_dry.jl:202-211,
-// with the half step k = 0.5*dt of its move! and accelerate! (:148-159):
-//   CD_KICK_MOVE  accelerate! then move!: fluid v += k (a + g); a = 0 for
-//                 every particle; fluid x += k v
-//   CD_MOVE       move!: a = 0; fluid x += k v
-//   CD_KICK       accelerate!: fluid v += k (a + g)
-// The continuity find_pressure! between them is SPH_OP_FIND_PRESSURE_CONTINUITY.
-__global__ __launch_bounds__(256) void k_cd_unary(int stage, const int* meta, double* cols,
-                                                  long long cap, const SysDesc* __restrict__ sysd,
-                                                  const int* __restrict__ sysid)
+// The accelerate! that ends the time loop of examples/collapse_dry.jl:202-211,
+// with the half step k = 0.5*dt (:155-159): fluid v += k (a + g).  The other
+// unary stages of the loop run in the key passes of its builds (cells.hip).
+__global__ __launch_bounds__(256) void k_cd_kick(const int* meta, double* cols, long long cap,
+                                                 const SysDesc* __restrict__ sysd,
+                                                 const int* __restrict__ sysid)
 {
     const int n = meta[META_N];
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
+    if (UCOL(cols, cap, C_TYPE, i) != 0.0) return;
     const Phys& ph = sysd[sysid[i]].ph;
     const double k = 0.5 * ph.dt;
-    const bool fluid = UCOL(cols, cap, C_TYPE, i) == 0.0;
-    double v[3];
-    for (int d = 0; d < 3; ++d) {
-        v[d] = UCOL(cols, cap, C_VX + d, i);
-        if (fluid && stage != CD_MOVE) {
-            v[d] = v[d] + k * (UCOL(cols, cap, C_AX + d, i) + ph.g[d]);
-            UCOL(cols, cap, C_VX + d, i) = v[d];
-        }
-    }
-    if (stage == CD_KICK) return;
-    for (int d = 0; d < 3; ++d) {
-        UCOL(cols, cap, C_AX + d, i) = 0.0;
-        if (fluid) UCOL(cols, cap, C_X + d, i) = UCOL(cols, cap, C_X + d, i) + k * v[d];
-    }
+    for (int d = 0; d < 3; ++d)
+        UCOL(cols, cap, C_VX + d, i) =
+            UCOL(cols, cap, C_VX + d, i) + k * (UCOL(cols, cap, C_AX + d, i) + ph.g[d]);
 }
 
 // ----------------------------------------------------------- reductions --
@@ -623,11 +609,11 @@ void enqueue_prho2(sph_system* s)
     k_prho2<<<nblk(s->n), 256, 0, s->stream>>>(s->meta, s->cols[s->cur], s->cap, s->prho2);
 }
 
-void enqueue_cd_unary(sph_system* s, int stage)
+void enqueue_cd_kick(sph_system* s)
 {
     if (s->n <= 0) return;
-    k_cd_unary<<<nblk(s->n), 256, 0, s->stream>>>(stage, s->meta, s->cols[s->cur], s->cap, s->sysd,
-                                                 sysid_col(s));
+    k_cd_kick<<<nblk(s->n), 256, 0, s->stream>>>(s->meta, s->cols[s->cur], s->cap, s->sysd,
+                                                sysid_col(s));
 }
 
 void enqueue_kick_drift(sph_system* s)
