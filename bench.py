@@ -468,8 +468,8 @@ def main():
                     "not in this run")
         return {
             "bound": "valu",
-            "ceiling": "vector ALU: the pair kernels issue no MFMA (the field's 'mfma' does not "
-                       "apply); peak is the published "
+            "ceiling": "vector ALU: the matrix cores only filter the candidates (the field's "
+                       "'mfma' does not apply); peak is the published "
                        f"{'packed FP32' if prec == 'mixed' else 'FP64'} vector rate",
             "kernel": name,
             "achieved": achieved,

@@ -300,7 +300,7 @@ int sph_autotune(sph_system* s, const sph_params* params, int* best);
 /* SPH_OPTION_GRAPH (default 0): sph_step / sph_batch_step capture the
  * kernels of one or two steps into a hipGraph once per call and replay it
  * for the call's steps, instead of enqueueing every kernel of every step
- * (about 25 launches per step).  Same bits; kernel profiling is off while
+ * (about eight launches per step).  Same bits; kernel profiling is off while
  * the graph replays. */
 #define SPH_OPTION_GRAPH 2
 int sph_set_option(sph_system* s, int option, int value);

@@ -29,9 +29,10 @@
 // one chunk per step, so its ring holds a single chunk (64 slots).
 //
 // Each chunk is handled in two phases:
-//   1. mask: lane (t, s) tests the chunk slots s + S*j (j < T) against
-//      target t and sets bit j of its T-bit mask for slot s + S*j -- or,
-//      after a density pass on the same cell list, loads that pass's mask.
+//   1. mask: the matrix cores (T >= 32, candidate test below) or lane
+//      (t, s) itself test the chunk slots s + S*j (j < T) against target t
+//      and set bit j of the lane's T-bit mask for slot s + S*j -- or, after
+//      a density pass on the same cell list, the lane loads that pass's mask.
 //      Interleaving the slices keeps the accepted counts of the lanes
 //      alike (neighbouring slots are neighbouring particles);
 //   2. interact: the chunk's accepted pairs are cut into runs spread over
@@ -46,8 +47,9 @@
 // RN(sqrt((d1*d1 + d2*d2) + d3*d3)) <= h.  sqrt is correctly rounded and
 // monotonic, so this equals s <= s_thr with s_thr = max{s : RN(sqrt(s)) <= h}
 // (computed on the host).  The FP64 kernels evaluate s without FMA
-// (-ffp-contract=off), i.e. bit-exactly as the reference.  The mixed
-// kernels evaluate |q|^2 - 2 p.q + |p|^2 in FP32 on tile-relative
+// (-ffp-contract=off), i.e. bit-exactly as the reference.  With T >= 32 both
+// modes filter on the matrix cores and settle the close pairs by that exact
+// test.  With T = 16 and 8 the mixed kernels evaluate |q|^2 - 2 p.q + |p|^2 in FP32 on tile-relative
 // coordinates (three FMAs per candidate): below s_thr (1 - BAND) the pair is
 // accepted, above s_thr (1 + BAND) rejected, and in between the exact FP64
 // test decides, so their neighbour sets (and masks) are the reference's
