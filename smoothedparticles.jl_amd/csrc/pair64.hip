@@ -25,14 +25,17 @@ __device__ inline double sqrt_pair(double s)
 }
 
 // n / d by Newton's iteration from the hardware's reciprocal and a residual
-// correction (Markstein), without the library's scaling of the operands.
+// correction (Markstein), without the library's scaling of the operands.  The
+// fixup puts the quotients of zeros, infinities and NaN right, where the
+// iteration makes NaN of all of them (5.76M particles 12.88 -> 12.71 ms, within
+// the noise).
 __device__ inline double div_pair(double n, double d)
 {
     double y = __builtin_amdgcn_rcp(d);
     y = fma(fma(-d, y, 1.0), y, y);
     y = fma(fma(-d, y, 1.0), y, y);
     const double q = n * y;
-    return fma(fma(-d, q, n), y, q);
+    return __builtin_amdgcn_div_fixup(fma(fma(-d, q, n), y, q), d, n);
 }
 
 // LDS ring of kept candidates (FP64): positions only, or xy, (z, rho),

@@ -51,3 +51,36 @@ def test_small_and_zero_distances(dim, h):
     assert off("a", o.field("a")) <= 1e-11
     assert off("Drho", o.field("Drho")) <= 1e-12
     assert np.max(np.abs(g.get("rho0") / o.field("rho0") - 1.0)) <= 1e-12
+
+
+@pytest.mark.parametrize("field,value", [("rho", np.inf), ("rho", -1000.0), ("v", np.inf),
+                                         ("v", -np.inf), ("v", np.nan)])
+def test_non_finite_quotients(field, value):
+    """One particle with an infinite density (its pairs' viscous quotients are
+    0), one that makes the mean density of a pair 0 (infinite quotients), or a
+    velocity that is no number: the accelerations are finite, infinite and NaN
+    where the oracle's are, the finite ones within 1e-11 of the largest."""
+    rng = np.random.default_rng(11)
+    n, h = 200, 0.5
+    x = 0.05 + 0.9 * rng.random((n, 3))
+    v = rng.normal(size=(n, 3))
+    rho = np.full(n, 1000.0)
+    P = 1.0e4 * rng.normal(size=n)
+    if field == "rho":
+        rho[7] = value
+    else:
+        v[7, 0] = value
+    kw = dict(m=1.0, rho0=1000.0, c=50.0, alpha=0.05, hs=h / 2.0, mu=0.0, nu=0.0, dt=1e-5)
+    g = sp.ParticleSystem(sp.Box(0, 0, 0, 1, 1, 1), h, "fp64")
+    g.add_particles(x, v=v, rho=rho, P=P, type=np.zeros(n))
+    o = O.OracleSystem(h, np.zeros(3), np.ones(3))
+    o.load(x, v, rho, P, np.zeros(n))
+    assert sp.create_cell_list(g) == o.create_cell_list()
+    sp.apply(g, sp.internal_force, **kw)
+    o.internal_force(**kw)
+    got, want = g.get("a"), o.field("a")
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[~fin & ~np.isnan(want)], want[~fin & ~np.isnan(want)])
+    if fin.any():
+        assert np.max(np.abs(got[fin] - want[fin])) <= 1e-11 * np.max(np.abs(want[fin]))
