@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -224,9 +225,10 @@ struct Pinned {
     hipEvent_t ev[PIN_PARTS] = {};
 };
 
-// (on the heap: handles may be destroyed while the process ends)
+// (the lock is on the heap: handles may be destroyed while the process ends)
 std::mutex& pin_mu = *new std::mutex;
-std::vector<Pinned*>& pin_idle = *new std::vector<Pinned*>;
+Pinned* pin_idle[PIN_KEEP];
+size_t pin_nidle = 0;
 int pin_handles = 0;
 
 void pin_free(Pinned* p)
@@ -243,15 +245,16 @@ Pinned* pin_take(int device, size_t bytes)
 {
     {
         std::lock_guard<std::mutex> lock(pin_mu);
-        for (size_t i = 0; i < pin_idle.size(); ++i) {
+        for (size_t i = 0; i < pin_nidle; ++i) {
             Pinned* p = pin_idle[i];
             if (p->device == device && p->bytes >= bytes) {
-                pin_idle.erase(pin_idle.begin() + (long)i);
+                pin_idle[i] = pin_idle[--pin_nidle];
                 return p;
             }
         }
     }
-    Pinned* p = new Pinned;
+    Pinned* p = new (std::nothrow) Pinned;
+    if (!p) return nullptr;
     p->bytes = bytes;
     p->device = device;
     hipError_t e = hipHostMalloc((void**)&p->mem, bytes, hipHostMallocDefault);
@@ -270,8 +273,8 @@ void pin_give(Pinned* p)
 {
     {
         std::lock_guard<std::mutex> lock(pin_mu);
-        if (pin_handles > 0 && pin_idle.size() < PIN_KEEP) {
-            pin_idle.push_back(p);
+        if (pin_handles > 0 && pin_nidle < PIN_KEEP) {
+            pin_idle[pin_nidle++] = p;
             return;
         }
     }
@@ -280,13 +283,9 @@ void pin_give(Pinned* p)
 
 void pin_handle(int change)
 {
-    std::vector<Pinned*> drop;
-    {
-        std::lock_guard<std::mutex> lock(pin_mu);
-        pin_handles += change;
-        if (pin_handles == 0) drop.swap(pin_idle);
-    }
-    for (Pinned* p : drop) pin_free(p);
+    std::lock_guard<std::mutex> lock(pin_mu);
+    pin_handles += change;
+    while (pin_handles == 0 && pin_nidle > 0) pin_free(pin_idle[--pin_nidle]);
 }
 
 // Copies `bytes` from device memory to the caller's array; the stream has
