@@ -32,6 +32,7 @@
 // 100 us, 30 us with these five; the 5.75M-particle dam break's took 560 us,
 // 390 us now (no permutation written and read back, the fluid's acceleration
 // left out, no pass for the tiles' boxes).
+#include "brick.h"
 #include "scan_kernels.h"
 #include "sph_internal.h"
 
@@ -465,38 +466,6 @@ __device__ inline void remove_seq(int s, int cells_total, const int* sc, const i
     }
 }
 
-// Local cell at rank lr of a system in brick order: the grid is cut into
-// bricks of BX x BY x BZ cells (BZ = 1 in 2D), the bricks are numbered x
-// fastest, then y, then z, and the cells of a brick x fastest; the bricks
-// on the far faces are cut to the grid, so the ranks are 0 .. key_max - 1.
-// The tile table follows this order: each XCD walks a contiguous share of
-// it, and the tiles it has in flight then cover a compact block of cells
-// whose neighbour cells (the candidates) are few enough to stay in its L2,
-// where a row-major order spreads them over whole rows of the grid.
-constexpr int BRICK_X = 4, BRICK_Y = 4, BRICK_Z = 4, BRICK_2D = 8;
-
-__device__ inline int brick_cell(const Geo& g, int lr)
-{
-    const int bx = g.L3 > 1 ? BRICK_X : BRICK_2D;
-    const int by = g.L3 > 1 ? BRICK_Y : BRICK_2D;
-    const int bz = g.L3 > 1 ? BRICK_Z : 1;
-    const int layer = bz * g.L1 * g.L2;  // a layer of bricks (the last may be thinner)
-    const int kz = lr / layer;
-    const int hz = min(bz, g.L3 - kz * bz);
-    int r = lr - kz * layer;
-    const int row = by * g.L1 * hz;      // a row of bricks
-    const int ky = r / row;
-    const int hy = min(by, g.L2 - ky * by);
-    r -= ky * row;
-    const int brick = bx * hy * hz;
-    const int kx = r / brick;
-    const int wx = min(bx, g.L1 - kx * bx);
-    r -= kx * brick;
-    const int iz = r / (wx * hy), q = r - iz * (wx * hy);
-    const int iy = q / wx, ix = q - iy * wx;
-    return kx * bx + ix + g.L1 * ((ky * by + iy) + g.L2 * (kz * bz + iz));
-}
-
 // 64-candidate chunks one target of cell c walks: the pair kernels
 // concatenate the cell's stencil ranges and cut the list into chunks of 64.
 template <int ROWS>
@@ -553,7 +522,7 @@ __global__ __launch_bounds__(256) void k_tile_table(
         words[k] = 0;
         if (r < ncells) {
             const SysDesc& d = sysd[cell_sys[r]];
-            const int lc = brick_cell(d.g, r - d.cell_base);
+            const int lc = brick_cell(d.g.L1, d.g.L2, d.g.L3, r - d.cell_base);
             const int c = d.cell_base + lc;
             const int n = cell_start[c + 1] - cell_start[c];
             cell[k] = c;
