@@ -603,9 +603,12 @@ static void enqueue_tile_table(sph_system* s, int removal)
     s->queue_used = 0;
 }
 
-// The tile table of the current cell list for another tile size.
+// The tile table of the current cell list for another tile size.  A batch
+// that holds no system (every one retired, or none added yet) has no cells, no
+// tiles and maybe no arrays for them.
 void enqueue_tiles(sph_system* s)
 {
+    if (s->cells_total == 0) return;
     const int nstat = (int)scan_state_needed(s->cells_cap);
     k_reset_scans<<<nblocks(nstat, 256), 256, 0, s->stream>>>(s->scan_state, nstat, s->meta);
     enqueue_tile_table(s, 0);
