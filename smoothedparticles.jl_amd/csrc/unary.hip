@@ -14,7 +14,8 @@ namespace sph {
 // ------------------------------------------------------------ operators --
 // A handle of one system passes its parameters by value (one != 0): the
 // operators of a program's loop come with different parameters call by call,
-// and an upload of its own cost each call a launch.
+// and an upload of its own cost each call a launch.  With several systems the
+// call's parameters are slot 0's and go to the device first.
 __global__ __launch_bounds__(256) void k_unary(int op, const int* meta, double* cols,
                                                long long cap, const SysDesc* __restrict__ sysd,
                                                const int* __restrict__ sysid, int one, Phys ph1)
@@ -598,6 +599,7 @@ void enqueue_unary(sph_system* s, int op)
 {
     if (s->n <= 0) return;
     const int one = s->sys_host.size() == 1;
+    if (!one) enqueue_params0(s);
     k_unary<<<nblk(s->n), 256, 0, s->stream>>>(op, s->meta, s->cols[s->cur], s->cap, s->sysd,
                                               sysid_col(s), one,
                                               one ? s->sys_host[0].ph : Phys{});
