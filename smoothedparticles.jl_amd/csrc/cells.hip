@@ -488,7 +488,8 @@ __device__ inline int cell_chunks(const SysDesc& d, const int* cell_start, int l
 // words are scanned together, by two waves of each block (chained blocks).  One
 // cell per thread: a small grid's table waits on one cell's loads and divisions
 // (1.5k cells 10.5 -> 7.0 us against four), a large one's chain is longer (93k
-// cells 24 -> 31 us of a 6.4 ms step).  The first block also clears the tile queues and replays the removals.
+// cells 24 -> 31 us of a 6.4 ms step).  The first block also clears the tile queues and, at
+// its end, replays the removals.
 static constexpr int TT_CELLS = 1;
 static constexpr int TT_TILE = 256 * TT_CELLS;
 
@@ -504,12 +505,7 @@ __global__ __launch_bounds__(256) void k_tile_table(
     __shared__ int with_tiles;
     if (threadIdx.x == 0) with_tiles = 0;
     const int b = chain_ticket(ticket);  // (a block barrier)
-    if (b == 0) {
-        if (threadIdx.x < NQUEUE_SETS * QSET / QSTRIDE) queue[threadIdx.x * QSTRIDE] = 0;
-        if (removal && meta[META_NREM] != 0)
-            for (int s = threadIdx.x; s < nsys; s += 256)
-                remove_seq(s, ncells, sc, cell_start, ref, inv);
-    }
+    if (b == 0 && threadIdx.x < NQUEUE_SETS * QSET / QSTRIDE) queue[threadIdx.x * QSTRIDE] = 0;
     int cell[TT_CELLS], nt[TT_CELLS];
     long long words[TT_CELLS];  // of one tile
     unsigned tsum = 0;
@@ -569,6 +565,10 @@ __global__ __launch_bounds__(256) void k_tile_table(
             wrun += (unsigned long long)words[k];
         }
     }
+    // The replay is a serial chain of reads (15 ms for 100,000 particles that
+    // leave at once), so it comes last: no block of the scan waits for it.
+    if (b == 0 && removal && meta[META_NREM] != 0)
+        for (int s = threadIdx.x; s < nsys; s += 256) remove_seq(s, ncells, sc, cell_start, ref, inv);
 }
 
 // State words of the scans and the count of cells with tiles, cleared for a
