@@ -484,16 +484,11 @@ __device__ inline int cell_chunks(const SysDesc& d, const int* cell_start, int l
 // Tile table, in brick order: tile k of the cell c at rank r covers targets
 // cell_start[c] + k*T ...; its pair masks start at the mask words of the
 // tiles before it (chunks * T words each), its kept-candidate list at 64 / T
-// times that.  Each thread takes TT_CELLS consecutive ranks; tiles and mask
-// words are scanned together, by two waves of each block (chained blocks).  One
-// cell per thread: a small grid's table waits on one cell's loads and divisions
-// (1.5k cells 10.5 -> 7.0 us against four), a large one's chain is longer (93k
-// cells 24 -> 31 us of a 6.4 ms step).  The first block also clears the tile queues and, at
-// its end, replays the removals.
-static constexpr int TT_CELLS = 1;
-static constexpr int TT_TILE = 256 * TT_CELLS;
-
-template <int ROWS>
+// times that.  Each thread takes CELLS consecutive ranks; tiles and mask
+// words are scanned together, by two waves of each block (chained blocks).
+// The first block also clears the tile queues and, at its end, replays the
+// removals.
+template <int ROWS, int CELLS>
 __global__ __launch_bounds__(256) void k_tile_table(
     const SysDesc* __restrict__ sysd, const int* __restrict__ cell_sys, int ncells,
     const int* __restrict__ cell_start, int T, long long mask_cap, long long kept_cap, int4* tiles,
@@ -506,14 +501,14 @@ __global__ __launch_bounds__(256) void k_tile_table(
     if (threadIdx.x == 0) with_tiles = 0;
     const int b = chain_ticket(ticket);  // (a block barrier)
     if (b == 0 && threadIdx.x < NQUEUE_SETS * QSET / QSTRIDE) queue[threadIdx.x * QSTRIDE] = 0;
-    int cell[TT_CELLS], nt[TT_CELLS];
-    long long words[TT_CELLS];  // of one tile
+    int cell[CELLS], nt[CELLS];
+    long long words[CELLS];  // of one tile
     unsigned tsum = 0;
     unsigned long long wsum = 0;
     int ncell = 0;
 #pragma unroll
-    for (int k = 0; k < TT_CELLS; ++k) {
-        const int r = b * TT_TILE + (int)threadIdx.x * TT_CELLS + k;
+    for (int k = 0; k < CELLS; ++k) {
+        const int r = b * 256 * CELLS + (int)threadIdx.x * CELLS + k;
         cell[k] = nt[k] = 0;
         words[k] = 0;
         if (r < ncells) {
@@ -557,7 +552,7 @@ __global__ __launch_bounds__(256) void k_tile_table(
         }
     }
 #pragma unroll
-    for (int k = 0; k < TT_CELLS; ++k) {
+    for (int k = 0; k < CELLS; ++k) {
         const int cs = nt[k] > 0 ? cell_start[cell[k]] : 0;
         for (int t = 0; t < nt[k]; ++t) {
             tiles[trun++] = make_int4(cell[k], cs + t * T, (int)(unsigned)(wrun & 0xffffffffull),
@@ -582,18 +577,32 @@ __global__ __launch_bounds__(256) void k_reset_scans(unsigned long long* stat, i
 // ------------------------------------------------------------ host side --
 static inline unsigned nblocks(long long n, int b) { return (unsigned)((n + b - 1) / b); }
 
+// Cells per thread of the tile table.  A table's blocks pass their sums on one
+// after the other, ~12 ns each, so a large grid wants few blocks; a small one's
+// table waits on one thread's loads and divisions, so it wants one cell per
+// thread.  A build of 20,000 particles at 1 / 8 cells per thread, us: 10k cells
+// 45 / 57, 90k 66 / 72, 202k 80 / 77, 490k 112 / 81, 1M 146 / 96, 16M 982 / 409
+// (3D: 97k 69 / 87, 1M 156 / 112, 4M 348 / 207); 2, 4, 16 or 32 gain at most 12%
+// over the better of the two.
+constexpr int TT_FEW = 1, TT_MANY = 8;
+constexpr int TT_MANY_CELLS = 1 << 17;
+
+static inline int tt_cells(long long ncells) { return ncells > TT_MANY_CELLS ? TT_MANY : TT_FEW; }
+
 // State words of the build's scans, for `cells` buckets: the counts, tiles
-// and mask words of each block, then one ticket per scan.
-static inline int stat_blocks(long long cells) { return (int)(cells / TT_TILE) + 2; }
+// and mask words of each block (with the most blocks), then one ticket per scan.
+static inline int stat_blocks(long long cells) { return (int)(cells / (256 * TT_FEW)) + 2; }
 long long scan_state_needed(long long cells) { return 3ll * stat_blocks(cells) + 2; }
 
 static void enqueue_tile_table(sph_system* s, int removal)
 {
     const int ncells = (int)s->cells_total;
-    const unsigned nb = nblocks(ncells, TT_TILE);
+    const bool many = tt_cells(ncells) == TT_MANY;
+    const unsigned nb = nblocks(ncells, 256 * tt_cells(ncells));
     const int sb = stat_blocks(s->cells_cap);
     unsigned long long* stat = s->scan_state;
-    auto k = s->rows == 3 ? k_tile_table<3> : k_tile_table<9>;
+    auto k = s->rows == 3 ? (many ? k_tile_table<3, TT_MANY> : k_tile_table<3, TT_FEW>)
+                          : (many ? k_tile_table<9, TT_MANY> : k_tile_table<9, TT_FEW>);
     k<<<nb, 256, 0, s->stream>>>(s->sysd, s->cell_sys, ncells, s->cell_start, s->tile_T,
                                  s->masks ? s->mask_cap : 0,
                                  s->kept && (s->kept_rg || !s->periodic) ? s->kept_cap : 0,
