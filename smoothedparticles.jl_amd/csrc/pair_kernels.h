@@ -227,10 +227,17 @@ __device__ inline int lowest_bit(MaskT<T> m)
 // with carry per test took 448, and no LDS read per test.
 //
 // D is only a filter.  Coordinates are scaled by a power of two to
-// 512 <= h < 1024, so no half overflows or loses bits to underflow; the
-// halves keep 2^-21 of a value and the sum of 16 products in FP32 loses at
-// most 16 * 2^-23 of its largest partial sum (8 h^2): together below 2e-5 h^2.
-// A pair with |D| below TEST_BAND h^2 (twice that) is settled by the exact
+// 512 <= h < 1024, so no half overflows or loses bits to underflow.  Its error:
+// two halves of 11 bits, both cut, keep 2^-21 of a value; the sum of 16 products
+// in FP32 loses at most 16 * 2^-23 of its largest partial sum.  Relative to the
+// centre of a box no wider than a cell, a pair near the threshold has
+// |q|^2 + 2|p||q| <= 6.8 h^2 with cells of h and <= 9.7 h^2 with the cells of up
+// to 4/3 h of a periodic box three cells wide, so the error is below 2.1e-5 h^2
+// and below 3.0e-5 h^2 (the products 3e-6 and 5e-6, |q|^2 and the FP32 roundings
+// of its terms 4e-6, the rest the sum).  That is the worst case of every rounding
+// at once: an emulation over 2.4e7 pairs, half of them from the corners outwards,
+// gave 3.8e-6.
+// A pair with |D| below TEST_BAND h^2 (above both) is settled by the exact
 // FP64 predicate, as in the FP32 test; found by a minimum over the lane's 16
 // values per block, and looked for bit by bit only in blocks that hold one
 // (about one in twenty).  So the masks are the reference's sets, bit for bit
