@@ -632,6 +632,7 @@ PairCtx make_ctx(sph_system* s)
     c.kept_n = s->kept_n;
     c.mask_mode = MASK_TEST;
     c.masks_mixed = s->precision == SPH_MIXED;
+    c.device = s->device;
     return c;
 }
 

@@ -63,6 +63,7 @@
 
 #include <type_traits>
 
+#include "device_cache.h"
 #include "sph_internal.h"
 
 namespace sph {
@@ -969,28 +970,32 @@ __device__ inline void write_eos(const PairCtx& c, const SysDesc& d, int p, doub
 }
 
 // -------------------------------------------------------------- launch --
-// Blocks of a kernel that the current device holds at once (one-wave
-// blocks, static LDS).
-inline int resident_blocks(const void* kernel)
+// Blocks of a kernel that a device holds at once (one-wave blocks, static
+// LDS), 0 if it cannot be asked.  (Every device runs the one gfx950 build, so a
+// compute unit holds the same number on each.)
+inline int resident_blocks(const void* kernel, int device)
 {
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0) != hipSuccess ||
-        cus < 1 || per_cu < 1) {
+    int cus = 0, per_cu = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0) != hipSuccess) {
         (void)hipGetLastError();
-        return 256 * 8;
+        return 0;
     }
     return cus * per_cu;
 }
 
 // Launch a tile kernel with the blocks it can use: no more than there are
-// tiles (grid) and no more than run at once.
+// tiles (grid) and no more than run at once on the handle's device.
+static constexpr int RESIDENT_DEVICES = 64, RESIDENT_UNKNOWN = 256 * 8;
+
 template <auto Kernel, class... Args>
-inline void launch_resident(int grid, hipStream_t st, Args... args)
+inline void launch_resident(int grid, hipStream_t st, const PairCtx& c, Args... args)
 {
-    static const int fill = resident_blocks(reinterpret_cast<const void*>(Kernel));
-    Kernel<<<grid < fill ? grid : fill, 64, 0, st>>>(args...);
+    static DeviceCache<RESIDENT_DEVICES> cache;
+    const int fill = cache.get(c.device, RESIDENT_UNKNOWN, [](int device) {
+        return resident_blocks(reinterpret_cast<const void*>(Kernel), device);
+    });
+    Kernel<<<grid < fill ? grid : fill, 64, 0, st>>>(c, args...);
 }
 
 }  // namespace sph

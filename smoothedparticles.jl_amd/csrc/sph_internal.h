@@ -126,6 +126,7 @@ struct PairCtx {
     int overwrite;            // write instead of accumulate
     int only_flagged;         // skip systems whose pass_on is 0
     int loading;              // kernels of a loading pass: LOAD_* (the device decides, or known)
+    int device;               // the handle's device (read by the launcher)
 };
 
 // The equation of state a fused step's density pass applies: none,
