@@ -257,10 +257,16 @@ Pinned* pin_take(int device, size_t bytes)
     if (!p) return nullptr;
     p->bytes = bytes;
     p->device = device;
-    hipError_t e = hipHostMalloc((void**)&p->mem, bytes, hipHostMallocDefault);
+    // An event is recorded only on streams of the device that was current when
+    // it was made, and the caller's thread may have another one current.
+    int current = device;
+    hipError_t e = hipGetDevice(&current);
+    if (e == hipSuccess && current != device) e = hipSetDevice(device);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&p->mem, bytes, hipHostMallocDefault);
     if (e != hipSuccess) p->mem = nullptr;
     for (int i = 0; i < PIN_PARTS && e == hipSuccess; ++i)
         e = hipEventCreateWithFlags(&p->ev[i], hipEventDisableTiming);
+    if (current != device) (void)hipSetDevice(current);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         pin_free(p);
