@@ -312,7 +312,12 @@ int sph_set_option(sph_system* s, int option, int value);
 int sph_candidates(sph_system* s, int64_t* all, int64_t* fluid);
 
 /* Kernel timing with HIP events on the system's stream.  Kernel ids:
- * 0 cell build, 1 density pass, 2 force pass, 3 unary/integrator. */
+ * 0 cell build, 1 density pass, 2 force pass, 3 unary/integrator.
+ * In a fused step (sph_step, sph_batch_step) the unary work runs inside other
+ * kernels and counts into them: kick and drift, and collapse_dry's half steps
+ * and continuity EOS, into the next step's cell build, the EOS of the other
+ * schemes into the density pass.  Kernel 3 then holds the last integrator stage
+ * of each call only. */
 #define SPH_KERNEL_BUILD 0
 #define SPH_KERNEL_DENSITY 1
 #define SPH_KERNEL_FORCE 2

@@ -606,8 +606,8 @@ void prof_collect(sph_system* s)
 // costs (3D dam break, us per step at T = 64 / 32: 105k particles 674 / 468,
 // 311k 1190 / 825, 1.7M 4375 / 3970, 5.76M 14550 / 13790).  The mixed mode's
 // shorter walk gains from it only below 640k particles (105k 366 / 308, 842k
-// 1079 / 1114, 5.76M 6440 / 7540), where it would change FP32 roundings for
-// 15%; there it is left to autotuning.
+// 1079 / 1114, 5.76M 6440 / 7540); its default keeps its size there, and with
+// it its bits, and sph_autotune picks the faster one.
 int choose_tile(double occupancy, int precision)
 {
     const int cap = precision == SPH_MIXED ? 64 : 32;

@@ -959,7 +959,9 @@ __device__ inline void digest_write(const PairCtx& c, int p, unsigned long long 
 // The equation of state of particle p whose density rho the pass has just
 // formed: the expressions of SPH_OP_FIND_PRESSURE(_RHO0).  A kernel of its own
 // that read rho back took 43 us of a 5.75M-particle step and 4 of a small one's
-// 75; here it costs nothing measurable (the density kernel has no spills).
+// 75; here it costs nothing measurable since the matrix-core test freed the
+// registers for it (before, the density kernel spilled and this made its pass
+// ~80 us longer; now it spills no vector register).
 __device__ inline void write_eos(const PairCtx& c, const SysDesc& d, int p, double rho)
 {
     if (c.eos == EOS_NONE) return;

@@ -7,12 +7,7 @@
 
 namespace sph {
 
-static constexpr int SCAN_ITEMS = 16;
-static constexpr int SCAN_TILE = 256 * SCAN_ITEMS;
-
-// Three launches: per-block sums, one block
-// scanning the block sums, per-block scans plus offset.  V is unsigned or
-// unsigned long long.
+// Inclusive scan over a wave; V is unsigned or unsigned long long.
 template <class V>
 __device__ inline V wave_incl_scan(V v)
 {
@@ -41,7 +36,8 @@ __device__ inline V block_incl_scan(V v, V& total)
     return w + off;
 }
 
-// Chained scan, one launch: every block scans its own part and takes the sum
+// Chained scan, one launch (the single-pass scan with decoupled look-back of
+// Merrill and Garland, 2016): every block scans its own part and takes the sum
 // of the parts before it from their state words.  A state word holds a value
 // and, in its top two bits, whether it is the block's own sum or the sum up
 // to and including the block; it is written and read as one 64-bit atomic,
@@ -92,6 +88,11 @@ __device__ inline unsigned long long chain_prefix(unsigned long long* stat, int 
                            __HIP_MEMORY_SCOPE_AGENT);
     return before;
 }
+
+// Scan in three launches: per-block sums, one block scanning the block sums,
+// per-block scans plus offset.
+static constexpr int SCAN_ITEMS = 16;
+static constexpr int SCAN_TILE = 256 * SCAN_ITEMS;
 
 template <class Src>
 __global__ __launch_bounds__(256) void k_scan_reduce(Src src, int n, typename Src::V* part)

@@ -41,10 +41,9 @@ enum Meta {
     META_NREM = 2,    // particles removed by the last build
     META_NTILES = 3,  // tiles of the pair kernels
     META_NCELLS = 4,  // non-empty cells
-    META_QUEUE = 5,   // (unused; the pair kernels' tile queues are separate)
-    META_MASK_OK = 6, // the pair-mask buffer holds this cell list's masks
-    META_KEPT_OK = 7, // the kept-candidate buffer holds this cell list's lists
-    META_SLOTS = 8
+    META_MASK_OK = 5, // the pair-mask buffer holds this cell list's masks
+    META_KEPT_OK = 6, // the kept-candidate buffer holds this cell list's lists
+    META_SLOTS = 7
 };
 
 // Per-system counters on the device (SYSCNT_* ints per system).
