@@ -579,15 +579,17 @@ static inline unsigned nblocks(long long n, int b) { return (unsigned)((n + b - 
 
 // Cells per thread of the tile table.  A table's blocks pass their sums on one
 // after the other, ~12 ns each, so a large grid wants few blocks; a small one's
-// table waits on one thread's loads and divisions, so it wants one cell per
-// thread.  A build of 20,000 particles at 1 / 8 cells per thread, us: 10k cells
-// 45 / 57, 90k 66 / 72, 202k 80 / 77, 490k 112 / 81, 1M 146 / 96, 16M 982 / 409
-// (3D: 97k 69 / 87, 1M 156 / 112, 4M 348 / 207); 2, 4, 16 or 32 gain at most 12%
-// over the better of the two.
+// table waits on one thread's loads and divisions (nine rows of them in 3D), so
+// it wants one cell per thread.  A build of 20,000 particles with 1 / 8 cells per
+// thread, us: 2D 90k cells 66 / 72, 137k 72 / 73, 202k 81 / 76, 1M 146 / 96, 16M
+// 982 / 409; 3D 97k 69 / 87, 195k 83 / 87, 262k 91 / 90, 512k 120 / 101, 4M
+// 348 / 207; 2, 4, 16 or 32 gain at most 12% over the better of the two.
 constexpr int TT_FEW = 1, TT_MANY = 8;
-constexpr int TT_MANY_CELLS = 1 << 17;
 
-static inline int tt_cells(long long ncells) { return ncells > TT_MANY_CELLS ? TT_MANY : TT_FEW; }
+static inline int tt_cells(int rows, long long ncells)
+{
+    return ncells > (rows == 3 ? 1 << 17 : 1 << 18) ? TT_MANY : TT_FEW;
+}
 
 // State words of the build's scans, for `cells` buckets: the counts, tiles
 // and mask words of each block (with the most blocks), then one ticket per scan.
@@ -597,8 +599,9 @@ long long scan_state_needed(long long cells) { return 3ll * stat_blocks(cells) +
 static void enqueue_tile_table(sph_system* s, int removal)
 {
     const int ncells = (int)s->cells_total;
-    const bool many = tt_cells(ncells) == TT_MANY;
-    const unsigned nb = nblocks(ncells, 256 * tt_cells(ncells));
+    const int per = tt_cells(s->rows, ncells);
+    const bool many = per == TT_MANY;
+    const unsigned nb = nblocks(ncells, 256 * per);
     const int sb = stat_blocks(s->cells_cap);
     unsigned long long* stat = s->scan_state;
     auto k = s->rows == 3 ? (many ? k_tile_table<3, TT_MANY> : k_tile_table<3, TT_FEW>)

@@ -1,5 +1,5 @@
 """The tile table on both sides of the grid size from which a thread takes
-eight cells instead of one (2^17 cells): neighbour sets, orders and removals
+eight cells instead of one (2^17 cells in 2D, 2^18 in 3D): neighbour sets, orders and removals
 are the oracle's, with the last block full, nearly empty and cut inside a
 thread's cells."""
 import numpy as np
@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T", [8, 32])
 @pytest.mark.parametrize("cells", [(512, 256, 1), (131071, 1, 1), (131073, 1, 1), (513, 256, 1),
                                    (1, 133121, 1), (64, 64, 32), (65, 64, 32), (51, 52, 53),
+                                   (64, 64, 64), (65, 64, 64), (131071, 1, 3), (67, 71, 73),
                                    (1030, 1021, 1)])
 def test_both_tables(cells, T):
     n = 12000
