@@ -578,6 +578,7 @@ __device__ inline void tile32(const PairCtx& c, int tile, int out_col, bool load
     if constexpr (MFMA)
         test_targets<T>(mt, lane, fmaf(tg.x, tsc, tcx), fmaf(tg.y, tsc, tcy),
                         FLAT ? 0.0f : fmaf(tg.z, tsc, tcz), (float)(d.g.h * d.g.tscale));
+    const bool wide = filter_too_wide<ROWS, FLAT, PERIODIC>(box.z0, box.z1, d.g.h);
     __syncthreads();
     typename Op::Acc acc;
     Op::init(acc);
@@ -647,6 +648,10 @@ __device__ inline void tile32(const PairCtx& c, int tile, int out_col, bool load
                     const float4 a = lds.pos[rb + sl];
                     test_chunk<T>(mt, fmaf(a.x, tsc, tcx), fmaf(a.y, tsc, tcy),
                                   FLAT ? 0.0f : fmaf(a.z, tsc, tcz), sl >= fill - head, m, unsure);
+                    if (wide) {
+                        m = 0;
+                        unsure = slots_below<T>(s, fill - head);
+                    }
                 } else {
                     // slots shifted in from the highest bit down
                     unsigned min = 0, mout = 0;

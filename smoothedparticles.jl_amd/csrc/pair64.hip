@@ -534,6 +534,7 @@ __device__ inline void tile64(const PairCtx& c, int tile, bool load_masks, bool 
                         (float)((tg.y - tcy) * d.g.tscale),
                         FLAT ? 0.0f : (float)((tg.z - tcz) * d.g.tscale),
                         (float)(d.g.h * d.g.tscale));
+    const bool wide = filter_too_wide<ROWS, FLAT, PERIODIC>(box.z0, box.z1, d.g.h);
     __syncthreads();
     typename Op::Acc acc;
     Op::init(acc);
@@ -604,6 +605,10 @@ __device__ inline void tile64(const PairCtx& c, int tile, bool load_masks, bool 
                                   (float)((qxy.y - tcy) * d.g.tscale),
                                   FLAT ? 0.0f : (float)((qz - tcz) * d.g.tscale),
                                   sl >= fill - head, m, unsure);
+                    if (wide) {
+                        m = 0;
+                        unsure = slots_below<T>(s, fill - head);
+                    }
                     // near the threshold: the exact predicate of the reference
                     while (__any(unsure != 0)) {
                         if (unsure) {

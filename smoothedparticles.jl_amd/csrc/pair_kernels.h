@@ -403,6 +403,26 @@ __device__ inline void test_chunk(const TestTile<T>& tt, float x, float y, float
     m &= ~unsure;
 }
 
+// Whether a tile's box is wider than the filter's error bound covers.  Positions
+// are bounded by their cell on every axis but one: the z of a flat periodic
+// system is free, and in a batch with a 2D system that is not flat it counts.
+// The pairs of such a tile are all settled by the exact test.
+template <int ROWS, bool FLAT, bool PERIODIC, class V>
+__device__ inline bool filter_too_wide(V z0, V z1, double h)
+{
+    if constexpr (ROWS == 3 && PERIODIC && !FLAT) return (double)(z1 - z0) > h;
+    else return false;
+}
+
+// The bits of slice s's slots below n, the end of the list in this chunk.
+template <int T>
+__device__ inline MaskT<T> slots_below(int s, int n)
+{
+    constexpr int S = 64 / T;
+    const int k = n > s ? (n - s + S - 1) / S : 0;
+    return k >= T ? ~MaskT<T>(0) : (MaskT<T>(1) << k) - 1;
+}
+
 // --------------------------------------------------------- wave reductions --
 // Inclusive prefix sum of v over the wave's lanes, in six DPP steps: the
 // row shifts by 1, 2, 4 and 8 lanes scan each row of 16 lanes, then the
